@@ -775,6 +775,62 @@ __global__ void __launch_bounds__(256) gemv_wr_kernel(GemvArgs a, int N) {
   }
 }
 
+// M = 1 with an int8 A row (the O projection of a split-attention token, one
+// row through q3_gemm_nt_group_store): whole weight rows as gemv_wr_kernel,
+// R rows per wave, the A row and its scales straight from memory (no LDS,
+// no barrier).  LPG lanes of 16 bytes hold one K-group (16: group 256, 8:
+// group 128); their exact int32 sums are combined with DPP, the group terms
+// added in ascending order.  BSG: per-(row, K-group) B scales.  Bound by one
+// memory round trip: N / 4 workgroups instead of the MFMA tile kernel's
+// N / 16 (O, K = 2048 x 1024: 5.3 -> 2.7 us with cached operands).
+template <int KB, int LPG, int R, bool BSG>
+__global__ void __launch_bounds__(256) gemv_wr_plain_kernel(GemvArgs a, int N) {
+  constexpr int GPJ = 64 / LPG;  // K-groups per 1024 bytes
+  const int lane = threadIdx.x & 63;
+  const int8_t *ap = pin_sgpr(a.a), *bp = pin_sgpr(a.seg[0].b);
+  const float *asp = pin_sgpr(a.as), *bsp = pin_sgpr(a.seg[0].bs);
+  float *outp = pin_sgpr(a.seg[0].out);
+  const int64_t bs_ld = BSG ? pin_sgpr(a.bs_ld) : 0;
+  const bool add = a.seg[0].epi == EPI_ADD;
+  const int row0 = (static_cast<int>(blockIdx.x) * 4 + wave_id()) * R;
+  int4 av[KB], w[R][KB];
+  float asg[KB], bsn[R][BSG ? KB : 1], base[R];
+#pragma unroll
+  for (int j = 0; j < KB; ++j) {
+    av[j] = *reinterpret_cast<const int4 *>(ap + 1024 * j + 16 * lane);
+    asg[j] = asp[GPJ * j + lane / LPG];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int n = min(row0 + r, N - 1);
+#pragma unroll
+    for (int j = 0; j < KB; ++j)
+      w[r][j] = *reinterpret_cast<const int4 *>(bp + static_cast<int64_t>(n) * (1024 * KB) + 1024 * j + 16 * lane);
+#pragma unroll
+    for (int j = 0; j < (BSG ? KB : 1); ++j) bsn[r][j] = BSG ? bsp[n * bs_ld + GPJ * j + lane / LPG] : bsp[n];
+    base[r] = add ? outp[n] : 0.0f;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float out = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      int acc = sdot4(w[r][j].x, av[j].x, 0);
+      acc = sdot4(w[r][j].y, av[j].y, acc);
+      acc = sdot4(w[r][j].z, av[j].z, acc);
+      acc = sdot4(w[r][j].w, av[j].w, acc);
+      acc += lane_xor<1>(acc);
+      acc += lane_xor<2>(acc);
+      acc += lane_xor<4>(acc);
+      if constexpr (LPG == 16) acc += lane_xor<8>(acc);
+      const float p = __fmul_rn(__fmul_rn(static_cast<float>(acc), bsn[r][BSG ? j : 0]), asg[j]);
+#pragma unroll
+      for (int g = 0; g < GPJ; ++g) out = __fadd_rn(out, lane_read(p, g * LPG));
+    }
+    if (lane == 0 && row0 + r < N) outp[row0 + r] = add ? __fadd_rn(base[r], out) : out;
+  }
+}
+
 // Per (row, head) wave: the head epilogues of the Q/K/V projections
 // (kernels/norm_rope_quant.h:17-86, group_gemm.h:173-193), from f32 rows.
 __global__ void __launch_bounds__(256) qkv_heads_kernel(QkvHeadArgs a) {
@@ -1004,6 +1060,35 @@ int wr_rows(const GemvArgs &a, int ncols) {
   return R;
 }
 
+// One row with an int8 A row, plain or residual store, one segment: 1 weight
+// row per wave up to 2048 columns (256-512 workgroups), 2 above.
+bool wr_plain(const GemvArgs &a, int ncols) {
+  const int epi = a.seg[0].epi;
+  return a.M == 1 && a.pro == PRO_NONE && a.nseg == 1 && !a.part && !a.clear && ncols < 65536 && ncols % 8 == 0 &&
+         (epi == EPI_STORE || epi == EPI_ADD) && a.K % 1024 == 0 && a.K >= 1024 && a.K <= 3072 &&
+         (a.group == 256 || (a.group == 128 && a.K <= 2048)) &&
+         (reinterpret_cast<uintptr_t>(a.a) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.seg[0].b) & 15) == 0;
+}
+
+template <int KB, int LPG, bool BSG>
+hipError_t launch_wr_plain(const GemvArgs &a, int ncols, hipStream_t s) {
+  if (ncols <= 2048)
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 1, BSG>), dim3(ncols / 4), dim3(256), 0, s, a, ncols);
+  else
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 2, BSG>), dim3(ncols / 8), dim3(256), 0, s, a, ncols);
+  return hipGetLastError();
+}
+
+template <bool BSG>
+hipError_t wr_plain_launch(const GemvArgs &a, int ncols, hipStream_t s) {
+  if (a.group == 256) {
+    if (a.K == 1024) return launch_wr_plain<1, 16, BSG>(a, ncols, s);
+    if (a.K == 2048) return launch_wr_plain<2, 16, BSG>(a, ncols, s);
+    return launch_wr_plain<3, 16, BSG>(a, ncols, s);
+  }
+  return a.K == 1024 ? launch_wr_plain<1, 8, BSG>(a, ncols, s) : launch_wr_plain<2, 8, BSG>(a, ncols, s);
+}
+
 bool wr_launch(const GemvArgs &a, int ncols, hipStream_t s, hipError_t *err) {
   if (!wr_rows(a, ncols)) return false;
   const bool two = a.seg[0].epi == EPI_SWIGLU;
@@ -1115,6 +1200,7 @@ hipError_t launch_gemv(const GemvArgs &a, hipStream_t s) {
     hipError_t err = hipSuccess;
     if (wr_launch(a, ncols, s, &err)) return err;
   }
+  if (wr_plain(a, ncols)) return a.bs_ld ? wr_plain_launch<true>(a, ncols, s) : wr_plain_launch<false>(a, ncols, s);
   const bool two = a.seg[0].epi == EPI_SWIGLU;
   if (a.M > 16) {  // a batch of rows: plain A operand, no partials, 16-column tiles
     if (a.pro != PRO_NONE || a.part || !gemv_rows_supported(a.M, a.K, a.group, ncols)) return hipErrorInvalidValue;

@@ -471,6 +471,44 @@ bool head_consts(int heads, int kv_heads);
 bool down_qkv_attn_supported(const GemvArgs &d, const GemvArgs &g, const AttnArgs &a);
 hipError_t launch_down_qkv_attn(const GemvArgs &d, const GemvArgs &g, const AttnArgs &a, hipStream_t s);
 
+// ---- decode attention over many workgroups per sequence (k_attn_split.hip) --
+// Three launches: the new token's head epilogues and every block's scores;
+// P and P8.V of every block; the den/res chain and the output.  Rows are
+// independent sequences (row_pos set: row r at position row_pos[r], page table
+// table + r * ld_table) or one sequence of kv_len keys.
+struct SplitArgs {
+  int rows, heads, kv_heads;  // heads = 2 kv_heads, head_dim 128
+  uint32_t kv_len;
+  const int32_t *row_pos;
+  const uint16_t *table;
+  int64_t ld_table;
+  int max_blocks;  // key blocks of the longest row
+  // projection rows f32: fq [rows][ldq], fk / fv [rows][ldk]; gains, RoPE
+  // tables [position][64]
+  const float *fq, *fk, *fv;
+  int64_t ldq, ldk;
+  const float *nq, *nk, *cos_t, *sin_t;
+  float inv_hd, qk_scale;
+  int8_t *k, *v;  // page pools: the new token's rows are written
+  float *ks, *vs;
+  uint32_t page_tokens;
+  int64_t page_bytes, row_bytes, scale_page_bytes, scale_row_bytes;
+  int8_t *q8;  // written for the record
+  float *qs;
+  int64_t ldq8, ldqs;
+  int8_t *o8;
+  float *os;
+  int64_t ldo, ldos;
+  // workspace [rows][heads][ldb]: x 32 scores, block maximum, running maximum,
+  // psum, x 128 pv
+  float *ws_s, *ws_bmax, *ws_nmm, *ws_psum, *ws_pv;
+  int64_t ldb;
+};
+bool attn_split_supported(const SplitArgs &a);
+// whether a batch with these key blocks (longest row, all rows) takes it
+bool attn_split_batch(int64_t max_blocks, int64_t sum_blocks);
+hipError_t launch_attn_split(const SplitArgs &a, hipStream_t s);
+
 // ---- greedy pick over a logits row (main_big.cpp:300-322) ---------------
 hipError_t launch_argmax_logits(const float *logits, int vocab,
                                 int32_t *out_id, const int32_t *pos_dev,

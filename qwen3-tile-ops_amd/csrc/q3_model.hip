@@ -24,6 +24,17 @@
 #include "q3_kernels.h"
 #include "q3ops.h"
 
+namespace {
+// Fewest key blocks (32 keys) of a single decoding row for the split
+// attention: below, the fused launch's walk of up to two chunks is faster
+// (token at 1300 keys 789 against 861 us, 1600: 887 / 872, 2047: 951 / 882,
+// 4000: 1403 / 957).
+constexpr uint32_t kSplitMin1 = 49;
+// blocks (of every head) that the split attention's workspace holds at most:
+// 10.4 KB each with 16 heads
+constexpr int64_t kSplitMaxBlocks = 8192;
+}  // namespace
+
 struct q3_model {
   uint8_t *blob;
   q3_layout lay;
@@ -71,6 +82,13 @@ struct q3_model {
   // device's CUs (down_qkv_attn_supported checks the count)
   bool merge = true;
   uint32_t *xw = nullptr;
+  // decode attention over many workgroups per sequence (k_attn_split.hip):
+  // workspace for split_blocks key blocks (of every head); Q3_ATTN_SPLIT at
+  // open: 0 off, 1 wherever it applies (the tests), else by size
+  float *split_ws = nullptr;
+  int64_t split_blocks = 0;
+  bool split_always = false;
+  std::vector<uint8_t> page_use;  // q3_decode_batch: one flag per pool page
   // event timing of decode kernel classes (q3_model_set_kernel_timing)
   uint32_t kt_mask = 0;
   std::vector<hipEvent_t> kt_ev[Q3_KT_COUNT];  // start, end pairs
@@ -337,6 +355,57 @@ q3::GemvSeg gemv_seg(int n0, int n1, int epi, const int8_t *b, const float *bs, 
   return g;
 }
 
+// The split decode attention of `rows` sequences (row_pos: device positions and
+// tables; else one sequence of kv_len keys through the model's table), whose
+// projection rows are in the blob's q / k / v stage rows; ldb blocks per row.
+q3::SplitArgs split_args(const q3_model *m, const LayerPtrs &lp, int rows, uint32_t kv_len, int ldb) {
+  const q3_layout &y = m->lay;
+  const int64_t QW = static_cast<int64_t>(y.heads) * y.head_dim, KW = static_cast<int64_t>(y.kv_heads) * y.head_dim;
+  q3::SplitArgs a{};
+  a.rows = rows;
+  a.heads = static_cast<int>(y.heads);
+  a.kv_heads = static_cast<int>(y.kv_heads);
+  a.kv_len = kv_len;
+  a.table = m->ptab;
+  a.max_blocks = ldb;
+  a.fq = at<const float>(m, y.kQ);
+  a.fk = at<const float>(m, y.kK);
+  a.fv = at<const float>(m, y.kV);
+  a.ldq = QW;
+  a.ldk = KW;
+  a.nq = lp.nq;
+  a.nk = lp.nk;
+  a.cos_t = at<const float>(m, y.kCOS);
+  a.sin_t = at<const float>(m, y.kSIN);
+  a.inv_hd = 1.0f / static_cast<float>(y.head_dim);
+  a.qk_scale = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(y.head_dim)));
+  a.k = lp.kc;
+  a.v = lp.vc;
+  a.ks = lp.kcs;
+  a.vs = lp.vcs;
+  a.page_tokens = kPageTokens;
+  a.page_bytes = kPageTokens * KW;
+  a.row_bytes = KW;
+  a.scale_page_bytes = static_cast<int64_t>(kPageTokens) * y.kv_heads * 4;
+  a.scale_row_bytes = y.kv_heads * 4;
+  a.q8 = at<int8_t>(m, y.kQ8);
+  a.qs = at<float>(m, y.kQS);
+  a.ldq8 = QW;
+  a.ldqs = y.heads;
+  a.o8 = at<int8_t>(m, y.kO8);
+  a.os = at<float>(m, y.kOS);
+  a.ldo = QW;
+  a.ldos = y.heads;
+  const int64_t nb = static_cast<int64_t>(rows) * y.heads * ldb;  // <= heads * split_blocks
+  a.ws_pv = m->split_ws;
+  a.ws_s = a.ws_pv + nb * 128;
+  a.ws_bmax = a.ws_s + nb * 32;
+  a.ws_nmm = a.ws_bmax + nb;
+  a.ws_psum = a.ws_nmm + nb;
+  a.ldb = ldb;
+  return a;
+}
+
 // True when a chunk of `rows` runs on the decode-shaped kernels.
 bool small_path(const q3_layout &y, uint32_t rows) {
   const int H = static_cast<int>(y.hidden);
@@ -584,8 +653,13 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
         t.pf_kv_heads = 0;
       }
     }
+    // a long context: the projection on its own, then the attention's key
+    // blocks over every CU
+    const uint32_t nblocks = (pos + rows + 31) / 32;
+    const bool split = fuse && m->split_ws && nblocks <= m->split_blocks && (m->split_always || nblocks >= kSplitMin1);
+    if (split) ofuse = false;
     bool qkvfuse = false;
-    if (ofuse && m->qkvfuse) {
+    if (ofuse && !split && m->qkvfuse) {
       t.xin = m->xin;
       t.xerr = m->xerr;
       qkvfuse = q3::qkv_attn_supported(gq, t);
@@ -614,7 +688,7 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
         g.npart = static_cast<int>(y.heads);
         g.ld_part = H;
       }
-      if (m->merge && rows == 1) {
+      if (m->merge && rows == 1 && !split) {
         g.clear = m->xw;
         g.nclear = q3::kXwWords;
         if (!q3::gemv_clear_supported(g)) g.clear = nullptr, g.nclear = 0;
@@ -684,7 +758,9 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
       }
     }
     if (!do_tail) continue;
-    if (merged) {
+    if (split) {
+      Q3_HIP(q3::launch_attn_split(split_args(m, lp, 1, pos + rows, static_cast<int>(nblocks)), s));
+    } else if (merged) {
       KTimer kt(m, Q3_KT_ATTN_DECODE);
       Q3_HIP(q3::launch_down_qkv_attn(pend, gq, t, s));
     } else if (qkvfuse) {
@@ -1211,6 +1287,18 @@ extern "C" int q3_model_open(void *blob, const q3_layout *lay, void *stream, q3_
       return Q3_ERR_HIP;
     }
   }
+  m->page_use.resize(m->n_pages);
+  const char *split_env = std::getenv("Q3_ATTN_SPLIT");
+  m->split_always = split_env && std::atoi(split_env) == 1;
+  if (lay->heads == 2 * lay->kv_heads && !(split_env && std::atoi(split_env) == 0)) {
+    // without room for it the single-launch attention takes every length
+    m->split_blocks = std::min<int64_t>(kSplitMaxBlocks, static_cast<int64_t>(lay->seq) * m->n_pages);
+    if (hipMalloc(&m->split_ws, sizeof(float) * static_cast<size_t>(lay->heads) * m->split_blocks * (128 + 32 + 3)) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      m->split_ws = nullptr;
+    }
+  }
   m->bpos = reinterpret_cast<int32_t *>(m->bstate);
   m->btab = reinterpret_cast<uint16_t *>(m->bstate + m->btab_off);
   std::vector<uint16_t> &tab = m->htab;
@@ -1254,6 +1342,28 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
     if (static_cast<uint32_t>(pos[r]) / kPageTokens >= ld_table) return Q3_ERR_RANGE;
     for (uint32_t i = 0; i <= static_cast<uint32_t>(pos[r]) / kPageTokens; ++i)
       if (tables[static_cast<size_t>(r) * ld_table + i] >= m->n_pages) return Q3_ERR_RANGE;
+  }
+  // the split attention: when a row is long, the batch's blocks fit the
+  // workspace, and no row's write page is a page of another row (its launch
+  // that writes the new K/V rows also reads the others' pages)
+  int64_t max_blocks = 0, sum_blocks = 0;
+  for (uint32_t r = 0; r < n; ++r) {
+    max_blocks = std::max<int64_t>(max_blocks, pos[r] / 32 + 1);
+    sum_blocks += pos[r] / 32 + 1;
+  }
+  bool split = m->split_ws && n * max_blocks <= m->split_blocks &&
+               (m->split_always || q3::attn_split_batch(max_blocks, sum_blocks));
+  if (split) {
+    std::vector<uint8_t> &use = m->page_use;  // 1: written by a row
+    std::fill(use.begin(), use.end(), uint8_t{0});
+    for (uint32_t r = 0; r < n && split; ++r) {
+      uint8_t &u = use[tables[static_cast<size_t>(r) * ld_table + static_cast<uint32_t>(pos[r]) / kPageTokens]];
+      split = u == 0;
+      u = 1;
+    }
+    for (uint32_t r = 0; r < n && split; ++r)
+      for (uint32_t i = 0; i < static_cast<uint32_t>(pos[r]) / kPageTokens && split; ++i)
+        split = use[tables[static_cast<size_t>(r) * ld_table + i]] == 0;
   }
   const hipStream_t s = m->stream;
   {
@@ -1342,6 +1452,14 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.seg[1] = gemv_seg(QW, QW + KW, q3::EPI_STORE, lp.wk, lp.wks, kf, KW);
       g.seg[2] = gemv_seg(QW + KW, QW + 2 * KW, q3::EPI_STORE, lp.wv, lp.wvs, vf, KW);
       Q3_HIP(q3::launch_gemv(g, s));
+    }
+    if (gv && split) {  // the head epilogues are part of the split attention
+      q3::SplitArgs a = split_args(m, lp, M, 0, static_cast<int>(max_blocks));
+      a.row_pos = m->bpos;
+      a.table = m->btab;
+      a.ld_table = ld_table;
+      Q3_HIP(q3::launch_attn_split(a, s));
+    } else if (gv) {
       q3::QkvHeadArgs e;
       std::memset(&e, 0, sizeof(e));
       e.M = M;
@@ -1422,7 +1540,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       if (!q3::gemm_tile_supported(t, q3::EPI_QKV)) return Q3_ERR_UNSUPPORTED;
       Q3_HIP(q3::launch_gemm_tile(t, q3::EPI_QKV, s));
     }
-    {
+    if (!(gv && split)) {
       q3::AttnArgs t{};
       t.rows = M;
       t.heads = static_cast<int>(y.heads);
@@ -1699,6 +1817,7 @@ extern "C" int q3_model_close(q3_model *m) {
   if (m->xin) (void)hipFree(m->xin);
   if (m->xerr) (void)hipFree(m->xerr);
   if (m->xw) (void)hipFree(m->xw);
+  if (m->split_ws) (void)hipFree(m->split_ws);
   if (m->dgraph) (void)hipGraphExecDestroy(m->dgraph);
   if (m->packed) (void)hipFree(m->packed);
   for (int c = 0; c < Q3_KT_COUNT; ++c)

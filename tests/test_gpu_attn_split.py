@@ -1,0 +1,121 @@
+"""The split decode attention (k_attn_split.hip: a sequence's key blocks over
+many workgroups) at the edges of its blocks (32 keys), workgroups (4 blocks)
+and chain stages (16 blocks, 128 per pass), against the oracle in batches and
+against the single-launch attention for one row; and the one-row whole-row
+GEMM that its O projection takes."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import bits_equal, describe_diff
+from test_gpu_batch import LD_TABLE, make_case, run_batch_case
+from test_gpu_ops import dev, host, rand_gemm
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from q3ops import LM_LOGITS, ops  # noqa: E402
+from q3ops.layout import InitConfig, Layout, ModelShape, init_random_blob  # noqa: E402
+from q3ops.model import Model  # noqa: E402
+
+
+@pytest.mark.parametrize("edge,ld_table", [
+    ([0, 30, 31, 32, 33, 126, 127, 128, 129, 253], LD_TABLE),
+    ([0, 510, 512, 2047, 4095, 4096, 4140], 132),
+])
+def test_split_batch_matches_oracle(cuda, monkeypatch, edge, ld_table):
+    monkeypatch.setenv("Q3_ATTN_SPLIT", "1")
+    n = len(edge)
+    run_batch_case(cuda, n, *make_case(n, seed=700 + n, edge=edge, ld_table=ld_table))
+
+
+def test_split_batch_shared_write_page(cuda, monkeypatch):
+    """Rows that write into a page another row reads take the single launch,
+    whose K/V rows are all written first: same ids with the split asked for."""
+    lay, blob, ctx, tables, _, ids0 = make_case(5, seed=105)
+    tables, ctx = tables.copy(), ctx.copy()
+    tables[1], ctx[1] = tables[4], ctx[4] + 1  # row 1 reads row 4's new token
+    tables[1, (ctx[1] // 32):] = tables[4, (ctx[1] // 32):]
+    got = []
+    for split in ("0", "1"):
+        monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+        m = Model(lay, blob)
+        out = torch.zeros(5, dtype=torch.int32, device=cuda)
+        m.decode_batch(torch.from_numpy(ids0.copy()).to(cuda), ctx, tables, out)
+        got.append((host(out), m.stage("x", 5)))
+        m.close()
+    assert np.array_equal(got[0][0], got[1][0]) and bits_equal(got[0][1], got[1][1])
+
+
+def test_split_one_row_matches_fused(cuda, monkeypatch):
+    """One decoding row at every edge: logits, residual row and the page rows
+    equal the fused launch's, over a shuffled page table."""
+    shape = ModelShape(layers=2, vocab=1024, seq=32, max_seq=4352)
+    lay = Layout(shape)
+    blob = init_random_blob(lay, InitConfig(n_prompt=1, n_gen=0, mode=0))
+    rng = np.random.default_rng(9)
+    o, ms = lay.offsets, lay.max_seq
+    for li in range(shape.layers):
+        base = o["kKV_BASE"] + li * o["kKV_STRIDE"]
+        for off in (0, o["kKV_VOFF"]):
+            n = ms * lay.kv_width
+            blob[base + off:base + off + n] = rng.integers(-127, 128, n, dtype=np.int8).view(np.uint8)
+            so = base + off + o["kKV_SOFF"]
+            sc = rng.uniform(0.002, 0.03, ms * lay.kv_heads).astype(np.float32)
+            blob[so:so + 4 * sc.size] = sc.view(np.uint8)
+    table = rng.permutation(ms // 32).astype(np.uint16)
+    ids = rng.integers(0, 1024, ms).astype(np.int32)
+    res = {}
+    for split in ("0", "1"):
+        monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+        m = Model(lay, blob)
+        m.set_page_table(table)
+        m.set_ids(ids)
+        for pos in (0, 30, 31, 32, 127, 128, 511, 512, 1567, 1568, 2047, 4095, 4096, 4351):
+            m.forward_chunk(pos, 1, LM_LOGITS, True)
+            res[split, pos] = [m.stage(nm, 1) for nm in ("logits", "x", "q8", "qs", "o8", "os")]
+        res[split, "kv"] = [m.kv_cache(li, ms)[nm] for li in range(2) for nm in ("kc", "ks", "vc", "vs")]
+        m.close()
+    for (split, what), v in res.items():
+        if split == "1":
+            for a, b in zip(v, res["0", what]):
+                assert bits_equal(a, b), (what, describe_diff(a, b))
+
+
+def test_split_generate_graph_replays(cuda, monkeypatch):
+    """The split decode steps captured in q3_generate's graph and replayed
+    equal the fused ones."""
+    shape = ModelShape(layers=2, vocab=1024, seq=64, max_seq=256)
+    lay = Layout(shape)
+    blob = init_random_blob(lay, InitConfig(n_prompt=100, n_gen=40, mode=0))
+    got = []
+    for split in ("0", "1"):
+        monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+        s = torch.cuda.Stream()
+        m = Model(lay, blob, stream=s)
+        m.set_ctrl(100, 40, 0)
+        for _ in range(3):
+            m.generate()
+            got.append(m.ids()[:140])
+        m.close()
+    assert all(np.array_equal(g, got[0]) for g in got[1:])
+
+
+@pytest.mark.parametrize("K,group", [(1024, 128), (1024, 256), (2048, 128), (2048, 256), (3072, 256)])
+@pytest.mark.parametrize("N", [128, 2048, 2176])
+@pytest.mark.parametrize("per_group", [False, True])
+def test_one_row_whole_row_gemm(cuda, K, group, N, per_group):
+    rng = np.random.default_rng(K + N + group)
+    a, as_, b, bs = rand_gemm(rng, 1, K, N, group)
+    if per_group:
+        bs = rng.uniform(1e-3, 1e-1, (N, K // group)).astype(np.float32)
+    ref = (oracle.gemm_nt_group_bg if per_group else oracle.gemm_nt_group)(a, as_, b, bs, group)
+    out = torch.zeros((1, N), dtype=torch.float32, device=cuda)
+    ops.gemm_nt_group_store(dev(a), dev(as_), dev(b), dev(bs), out, group)
+    assert bits_equal(host(out), ref), describe_diff(host(out), ref)
+    x = rng.normal(size=(1, N)).astype(np.float32)
+    xt = dev(x)
+    ops.gemm_nt_group_store(dev(a), dev(as_), dev(b), dev(bs), None, group, add=xt)
+    assert bits_equal(host(xt), (ref + x).astype(np.float32))
