@@ -847,6 +847,7 @@ __global__ void __launch_bounds__(256) qkv_heads_kernel(QkvHeadArgs a) {
   const float *nw;
   const float *cs;
   const float *sn;
+  if (h < a.q_heads && m < a.q_row0) return;
   if (h < a.q_heads) {
     src = a.q + static_cast<int64_t>(m) * a.ldq + h * 128;
     d = a.qd;

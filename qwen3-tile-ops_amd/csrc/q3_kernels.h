@@ -428,6 +428,7 @@ hipError_t launch_gemv(const GemvArgs &a, hipStream_t s);
 // RMSNorm + RoPE + quant (Q, K) or quant (V) into dense or paged int8.
 struct QkvHeadArgs {
   int M, q_heads, kv_heads;
+  int q_row0;  // Q rows before it are left out
   const float *q, *k, *v;
   int64_t ldq, ldk;
   QDest qd, kd, vd;

@@ -124,7 +124,12 @@ thread_local const LaunchEvents *g_launch_events = nullptr;
 namespace {
 
 constexpr uint32_t kPageTokens = 32;
-constexpr int kMaxGemvRows = 16;
+// Rows of a chunk on the GEMVs with prologues (forward_small): each workgroup
+// rebuilds the int8 rows one after the other, ~1 us per row and launch, so
+// from 5 rows on the row kernels and plain GEMVs of the 17-64-row path are
+// faster (28 layers, us: 4 rows 1130 against 1169, 5 1217 / 1166, 8 1461 /
+// 1183, 16 2170 / 1207).
+constexpr int kMaxSmallRows = 4;
 
 int hip_status(hipError_t e) { return e == hipSuccess ? Q3_OK : Q3_ERR_HIP; }
 
@@ -410,7 +415,7 @@ q3::SplitArgs split_args(const q3_model *m, const LayerPtrs &lp, int rows, uint3
 bool small_path(const q3_layout &y, uint32_t rows) {
   const int H = static_cast<int>(y.hidden);
   const int QW = static_cast<int>(y.heads * y.head_dim);
-  return rows <= static_cast<uint32_t>(kMaxGemvRows) && q3::gemv_supported(static_cast<int>(rows), H, 256) &&
+  return rows <= static_cast<uint32_t>(kMaxSmallRows) && q3::gemv_supported(static_cast<int>(rows), H, 256) &&
          q3::gemv_supported(static_cast<int>(rows), QW, static_cast<int>(y.head_dim)) &&
          q3::gemv_supported(static_cast<int>(rows), static_cast<int>(y.inter), 256);
 }
@@ -838,11 +843,10 @@ int qkv_projections(q3_model *m, const LayerPtrs &lp, uint32_t pos, uint32_t row
   const float *cos_t = at<const float>(m, y.kCOS);
   const float *sin_t = at<const float>(m, y.kSIN);
   const float inv_hd = 1.0f / static_cast<float>(HD);
-  if (do_tail && tr0 == 0 && tr == rows && rows <= 64 &&
-      q3::gemv_rows_supported(static_cast<int>(rows), H, 256, QW + 2 * KW)) {
+  if (do_tail && rows <= 64 && q3::gemv_rows_supported(static_cast<int>(rows), H, 256, QW + 2 * KW)) {
     // up to 64 rows: Q | K | V rows in f32 on the GEMV tiles, then the head
-    // epilogues of every (row, head) (Q into q8/qs, K and V into the page
-    // slots of positions pos + row)
+    // epilogues of every (row, head) (Q of the tail rows into q8/qs, K and V
+    // into the page slots of positions pos + row)
     float *qf = at<float>(m, y.kQ), *kf = at<float>(m, y.kK), *vf = at<float>(m, y.kV);
     q3::GemvArgs g = gemv_args(static_cast<int>(rows), H, 256);
     g.a = h8;
@@ -857,6 +861,7 @@ int qkv_projections(q3_model *m, const LayerPtrs &lp, uint32_t pos, uint32_t row
     q3::QkvHeadArgs e;
     std::memset(&e, 0, sizeof(e));
     e.M = static_cast<int>(rows);
+    e.q_row0 = static_cast<int>(tr0);
     e.q_heads = static_cast<int>(y.heads);
     e.kv_heads = static_cast<int>(y.kv_heads);
     e.q = qf;

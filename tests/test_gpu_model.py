@@ -190,6 +190,24 @@ def test_cfg0_prompt_chunk_sizes(cuda, seq):
     m.close()
 
 
+@pytest.mark.parametrize("seq", [3, 4, 5, 8, 16])
+def test_cfg0_short_chunks(cuda, seq):
+    """The 40-token prompt in chunks of 3 to 16 rows, on both sides of the
+    prologue GEMVs' row limit, with the last layer's tail on the last row
+    only: the reference's ids and logits, and its K/V rows."""
+    g = load_cfg("cfg0")
+    lay, blob = host_blob("cfg0", shape=ModelShape(layers=1, vocab=1024, seq=seq, max_seq=256))
+    m = Model(lay, blob)
+    for pos in range(0, 40, seq):
+        rows = min(seq, 40 - pos)
+        m.forward_chunk(pos, rows, LM_LOGITS, optimize_tail=True)
+    got = m.stage("logits", 1)[0]
+    assert int(np.argmax(got)) == int(g["generated"][0])
+    caches = m.kv_cache(0, 40)
+    assert not [p for st in ("kc", "ks", "vc", "vs") if (p := compare_stage(g, "f0_", st, caches[st]))]
+    m.close()
+
+
 def test_cfg2_full_depth(cuda, gold_meta):
     note("cfg2 28 layers, 32-token prefill, mode 1")
     lay, blob = host_blob("cfg2")
