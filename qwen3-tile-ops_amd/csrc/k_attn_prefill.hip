@@ -39,6 +39,15 @@
 // of a two-chunk LDS ring, the K operand rows and ks | vs straight into
 // registers.
 //
+// What bounds it: VALU issue (about 620 instructions per wave, block and 16
+// rows; the exps are 5 % of the time) and, with few workgroups, the serial
+// phases of a step (4.2 us for 8 blocks on an otherwise idle CU).  K rows and
+// scales of a chunk are loaded under phases 2 to 4 of the chunk before (after
+// phase 3 they cost 27 % of a long walk).  512 rows x 512 keys 15.2 us, 512 x
+// 3500 78 us, 301 x 2349 50 us, 2048 x 2048 112 us (before the early loads,
+// 32-bit offsets, immediate LDS offsets, the approximate reciprocal and the
+// corr = 1 path: 15.4, 94, 60 and 129 us).
+//
 // Layouts (lane = lc + 16 lg):
 //   S^T_j = K_j . Q^T with v_mfma_i32_16x16x64_i8, keys as the M dimension:
 //     lane holds s[kt][i] for key 16 kt + 4 lg + i, query row lc, so a
@@ -53,10 +62,12 @@
 //     lane (lc, lg) receives row lc, dims 4 lg..4 lg + 3 of the wave's tile.
 //   V stage  [32 keys][8 x 16 B], chunk c of key r at c ^ ((r & 3) | ((r >> 2) & 4)):
 //     the 8 keys a transposing read gathers land on 8 different chunks.
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
 
 #include "q3_device.h"
+#include "q3_epi.h"
 #include "q3_kernels.h"
 
 namespace q3 {
@@ -88,6 +99,7 @@ struct Lds {
   float bm[NI][QB][LDB];       // block maxima [item][row][block]
   float corr[NI][QB][LDB], psum[NI][QB][LDB], pmax[NI][QB][LDB];
   float cmax[NI][QB][8];       // |out| maxima of each 16-dim tile
+  float sc[CB][2 * KB];        // ks | vs of each wave's block
   uint64_t etab[32];
 };
 static_assert(sizeof(Lds<1>) <= 80 * 1024, "two single-block workgroups per CU");
@@ -247,7 +259,6 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
 
   // ---- this wave's copies of its block of chunk g ----
   v4i kop[2][2];  // K operand rows of the wave's block: [kt][64-byte k-step]
-  const int phys = lane & 7;
   // the page id of the wave's block of chunk g, held by lane 0: a kernel
   // argument for the first blk_page_n blocks, else a table load (per lane: a
   // wave-uniform load would be read into a scalar register at once, making
@@ -265,49 +276,44 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
     return p;
   };
   auto pg = [](uint32_t p) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(p), 0)); };
-  // in-page offsets fit in 32 bits (checked on the host)
-  const int rb = static_cast<int>(pa.row_bytes), srb = static_cast<int>(pa.scale_row_bytes);
+  // in-page offsets fit in 32 bits (checked on the host).  Every address is a
+  // wave-uniform base plus an unsigned 32-bit lane offset, which the loads
+  // take as they are (a signed offset costs a 64-bit add per load).
+  const uint32_t rb = static_cast<uint32_t>(pa.row_bytes), srb = static_cast<uint32_t>(pa.scale_row_bytes);
+  auto slot_of = [&](int g) { return static_cast<uint32_t>((g * CB + wave) * KB) & (pa.page_tokens - 1); };
   auto copy_v = [&](int g, uint32_t page) {
     if (g >= G || wave >= nb_of(1, g)) return;
-    const int slot0 = ((g * CB + wave) * KB) & (pa.page_tokens - 1);
-    const int8_t *vb = pa.v + static_cast<int64_t>(pg(page)) * pa.page_bytes + kvh * HD;
+    const int8_t *vb = pa.v + (static_cast<int64_t>(pg(page)) * pa.page_bytes + kvh * HD + slot_of(g) * rb);
     int8_t *dst = L.v[g & 1][wave];
+    // key 8 t + l3: vswz(key) = (l3 & 3) | (t & 2) << 1
+    const uint32_t l3 = static_cast<uint32_t>(lane) >> 3;
+    const uint32_t off = l3 * rb + (((static_cast<uint32_t>(lane) & 7) ^ (l3 & 3)) << 4);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int key = 8 * t + (lane >> 3);
-      const int off = (slot0 + key) * rb + ((phys ^ vswz(key)) << 4);
-      __builtin_amdgcn_global_load_lds(const_cast<int8_t *>(vb + off), to_lds(dst + t * 1024), 16, 0, 0);
+      const int8_t *src = vb + (8u * t * rb) + (t < 2 ? off : off ^ 64u);
+      __builtin_amdgcn_global_load_lds(const_cast<int8_t *>(src), to_lds(dst + t * 1024), 16, 0, 0);
     }
   };
   auto load_k = [&](int g, uint32_t page) {
     if (g >= G || wave >= nb_of(1, g)) return;
-    const int slot0 = ((g * CB + wave) * KB) & (pa.page_tokens - 1);
-    const int8_t *kb = pa.k + static_cast<int64_t>(pg(page)) * pa.page_bytes + kvh * HD;
+    const int8_t *kb = pa.k + (static_cast<int64_t>(pg(page)) * pa.page_bytes + kvh * HD + slot_of(g) * rb);
+    const uint32_t off = static_cast<uint32_t>(lc) * rb + 16u * static_cast<uint32_t>(lg);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
-        kop[kt][ks] = *reinterpret_cast<const v4i *>(kb + ((slot0 + 16 * kt + lc) * rb + 64 * ks + 16 * lg));
+        kop[kt][ks] = *reinterpret_cast<const v4i *>(kb + 16u * kt * rb + off + 64u * ks);
   };
-  // ks and vs of keys 16 kt + 4 lg + i of the wave's block, in registers
-  // (not staged through LDS by global_load_lds: a DS read of memory that an
-  // LDS DMA writes waits for every DMA in flight, i.e. for the next chunk's
-  // V copies)
-  float ksr[2][4], vsr[2][4];
+  // lane l < 32: ks of key l of the wave's block, lane 32 + l: vs of key l
+  // (one load; phase 1 spreads them through the wave's LDS slot.  Staging
+  // them by global_load_lds instead would make a DS read wait for every DMA
+  // in flight, i.e. for the next chunk's V copies)
+  float scv;
   auto load_sc = [&](int g, uint32_t page) {
     if (g >= G || wave >= nb_of(1, g)) return;
-    const int slot0 = ((g * CB + wave) * KB) & (pa.page_tokens - 1);
-    const int64_t sp = static_cast<int64_t>(pg(page)) * pa.scale_page_bytes + kvh * 4;
-    const int8_t *kb = reinterpret_cast<const int8_t *>(pa.ks) + sp;
-    const int8_t *vb = reinterpret_cast<const int8_t *>(pa.vs) + sp;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int off = (slot0 + 16 * kt + 4 * lg + i) * srb;
-        ksr[kt][i] = *reinterpret_cast<const float *>(kb + off);
-        vsr[kt][i] = *reinterpret_cast<const float *>(vb + off);
-      }
+    const int64_t sp = static_cast<int64_t>(pg(page)) * pa.scale_page_bytes + kvh * 4 + slot_of(g) * srb;
+    const int8_t *sb = reinterpret_cast<const int8_t *>(lane < 32 ? pa.ks : pa.vs) + sp;
+    scv = *reinterpret_cast<const float *>(sb + (static_cast<uint32_t>(lane) & 31) * srb);
   };
 
   // ---- prologue: chunk 0 in flight, exp table, Q operands of both items ----
@@ -357,7 +363,9 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
       const int gp = g - 1;
       const int nbp = nb_of(it4, gp);
       const int8_t *vbase = &L.v[gp & 1][0][0];
-      for (int b0 = 0; b0 < nbp; b0 += 4) {
+      static_for<CB / 4>([&](auto B4) {
+        constexpr int b0 = 4 * decltype(B4)::value;
+        if (b0 >= nbp) return;
         float4 c4, p4, s4;
         v2i vt[4];
         long pbv[4];
@@ -375,25 +383,28 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
           // (one asm statement: the values exist only after its wait, and the
           // early-clobbered outputs keep the addresses intact until issued)
           auto la = [](const void *p) { return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)); };
+          // Three base addresses; blocks and arrays by immediate offset.
+          constexpr int kPmax = offsetof(Lds<1>, pmax) - offsetof(Lds<1>, corr);
+          constexpr int kPsum = offsetof(Lds<1>, psum) - offsetof(Lds<1>, corr);
           asm volatile(
-              "ds_read_b128 %0, %11\n\t"
-              "ds_read_b128 %1, %12\n\t"
-              "ds_read_b128 %2, %13\n\t"
-              "ds_read_b64_tr_b8 %3, %14\n\t"
-              "ds_read_b64_tr_b8 %4, %15\n\t"
-              "ds_read_b64_tr_b8 %5, %16\n\t"
-              "ds_read_b64_tr_b8 %6, %17\n\t"
-              "ds_read_b64 %7, %18\n\t"
-              "ds_read_b64 %8, %19\n\t"
-              "ds_read_b64 %9, %20\n\t"
-              "ds_read_b64 %10, %21\n\t"
+              "ds_read_b128 %0, %11 offset:%c14\n\t"
+              "ds_read_b64_tr_b8 %3, %12 offset:%c17\n\t"
+              "ds_read_b64 %7, %13 offset:%c21\n\t"
+              "ds_read_b64_tr_b8 %4, %12 offset:%c18\n\t"
+              "ds_read_b64 %8, %13 offset:%c22\n\t"
+              "ds_read_b64_tr_b8 %5, %12 offset:%c19\n\t"
+              "ds_read_b64 %9, %13 offset:%c23\n\t"
+              "ds_read_b64_tr_b8 %6, %12 offset:%c20\n\t"
+              "ds_read_b64 %10, %13 offset:%c24\n\t"
+              "ds_read_b128 %1, %11 offset:%c15\n\t"
+              "ds_read_b128 %2, %11 offset:%c16\n\t"
               "s_waitcnt lgkmcnt(0)"
               : "=&v"(c4), "=&v"(p4), "=&v"(s4), "=&v"(vt[0]), "=&v"(vt[1]), "=&v"(vt[2]), "=&v"(vt[3]),
                 "=&v"(pbv[0]), "=&v"(pbv[1]), "=&v"(pbv[2]), "=&v"(pbv[3])
-              : "v"(la(&L.corr[sl(it4)][lc][b0])), "v"(la(&L.pmax[sl(it4)][lc][b0])),
-                "v"(la(&L.psum[sl(it4)][lc][b0])), "v"(la(vq)), "v"(la(vq + KB * HD)), "v"(la(vq + 2 * KB * HD)),
-                "v"(la(vq + 3 * KB * HD)), "v"(la(&L.p8[sl(it4)][b0][lane])), "v"(la(&L.p8[sl(it4)][b0 + 1][lane])),
-                "v"(la(&L.p8[sl(it4)][b0 + 2][lane])), "v"(la(&L.p8[sl(it4)][b0 + 3][lane]))
+              : "v"(la(&L.corr[0][lc][0])), "v"(la(vbase + v_tr_off)), "v"(la(&L.p8[0][0][lane])),
+                "n"(4 * b0), "n"(kPmax + 4 * b0), "n"(kPsum + 4 * b0), "n"(b0 * KB * HD), "n"((b0 + 1) * KB * HD),
+                "n"((b0 + 2) * KB * HD), "n"((b0 + 3) * KB * HD), "n"(512 * b0), "n"(512 * (b0 + 1)),
+                "n"(512 * (b0 + 2)), "n"(512 * (b0 + 3))
               : "memory");
         } else {  // (16 waves: the asm form's outputs do not fit the registers)
           c4 = *reinterpret_cast<const float4 *>(&L.corr[sl(it4)][lc][b0]);
@@ -415,18 +426,32 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
           __builtin_memcpy(&va, &vt[b], sizeof(va));
           c[b] = __builtin_amdgcn_mfma_i32_16x16x32_i8(va, pbv[b], zero4(), 0, 0, 0);
         }
+        // (corr = 1 in every row of four whole blocks, the usual case late in
+        // a long walk: x * 1 = x)
+        const bool ones = __builtin_amdgcn_ballot_w64(
+                              !(__fmul_rn(__fmul_rn(crv[0], crv[1]), __fmul_rn(crv[2], crv[3])) == 1.0f)) == 0;
+        if (ones && b0 + 4 <= nbp) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          if (b0 + b < nbp) {
+          for (int b = 0; b < 4; ++b) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float part = __fmul_rn(static_cast<float>(c[b][i]), pmv[b]);
-              res[i] = __fadd_rn(__fmul_rn(res[i], crv[b]), part);
+            for (int i = 0; i < 4; ++i)
+              res[i] = __fadd_rn(res[i], __fmul_rn(static_cast<float>(c[b][i]), pmv[b]));
+            den = __fadd_rn(den, psv[b]);
+          }
+        } else {
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            if (b0 + b < nbp) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float part = __fmul_rn(static_cast<float>(c[b][i]), pmv[b]);
+                res[i] = __fadd_rn(__fmul_rn(res[i], crv[b]), part);
+              }
+              den = __fadd_rn(__fmul_rn(den, crv[b]), psv[b]);
             }
-            den = __fadd_rn(__fmul_rn(den, crv[b]), psv[b]);
           }
         }
-      }
+      });
       if (last_of(it4, gp)) {  // out = res * (1/den); |out| maximum of the tile's 16 dims
         ended = true;
         const bool extra = it4 ? IB.extra : IA.extra;
@@ -452,7 +477,20 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
     const int nbA = g < G ? nb_of(0, g) : 0, nbB = g < G ? nb_of(1, g) : 0;
     const int j = g * CB + wave;
     wait_vmcnt<0>();  // this wave's copies and K rows of chunk g
+    float vsr[2][4];  // vs of keys 16 kt + 4 lg + i (0 past kv_len: P is 0 there)
     if (wave < nbB) {
+      float *sc = L.sc[wave];
+      sc[lane] = j * KB + (lane & 31) < kv_len ? scv : 0.0f;
+      float4 ks4[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        ks4[kt] = *reinterpret_cast<const float4 *>(sc + 16 * kt + 4 * lg);
+        const float4 v4 = *reinterpret_cast<const float4 *>(sc + KB + 16 * kt + 4 * lg);
+        vsr[kt][0] = v4.x;
+        vsr[kt][1] = v4.y;
+        vsr[kt][2] = v4.z;
+        vsr[kt][3] = v4.w;
+      }
 #pragma unroll
       for (int it = 0; it < 2; ++it) {
         if (it == 1 || wave < nbA) {
@@ -464,7 +502,7 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
           for (int kt = 0; kt < 2; ++kt) {
             v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[kt][0], qop[it][0], zero4(), 0, 0, 0);
             acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[kt][1], qop[it][1], acc, 0, 0, 0);
-            const float kv[4] = {ksr[kt][0], ksr[kt][1], ksr[kt][2], ksr[kt][3]};
+            const float kv[4] = {ks4[kt].x, ks4[kt].y, ks4[kt].z, ks4[kt].w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               float x = static_cast<float>(acc[i]);
@@ -486,6 +524,12 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
           if (lg == 0) L.bm[sl(it)][lc][wave] = bmax;
         }
       }
+    }
+    // K rows and ks | vs of chunk g + 1 (their registers were last read
+    // above), under phases 2 to 4
+    if (g < G) {
+      load_k(g + 1, page);
+      load_sc(g + 1, page);
     }
     lds_barrier();  // B1(g)
 
@@ -515,6 +559,7 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
 
     // ---- V rows of chunk g + 1 (V(g - 1)'s half was last read before B1(g)) ----
     copy_v(g + 1, page);
+    page = page_of(g + 2);
 
     // ---- phase 2: prefix max of the block maxima, per item, in block order ----
     // (each wave folds up to its own block; all blocks only when the item's
@@ -525,19 +570,29 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
       const int nb = it ? nbB : nbA;
       float m = g == 0 ? -3.402823466e38f : m_run[it];
       const bool carry = (it ? nB : nA) > (g + 1) * CB;
-      const float *bmr = L.bm[sl(it)][lc];
+      float bmr[CB];
 #pragma unroll
-      for (int b = 0; b < CB; ++b)
-        if (b < min(wave, nb)) m = (m > bmr[b]) ? m : bmr[b];
+      for (int b = 0; b < CB; b += 4) {
+        const float4 b4 = *reinterpret_cast<const float4 *>(&L.bm[sl(it)][lc][b]);
+        bmr[b] = b4.x;
+        bmr[b + 1] = b4.y;
+        bmr[b + 2] = b4.z;
+        bmr[b + 3] = b4.w;
+      }
+#pragma unroll
+      for (int b = 0; b < CB; ++b) {
+        const float v = b < min(wave, nb) ? bmr[b] : m;
+        m = (m > v) ? m : v;
+      }
       m_prev[it] = m_mine[it] = m;
       if (wave < nb) {
-        m = (m > bmr[wave]) ? m : bmr[wave];
+        const float own = L.bm[sl(it)][lc][wave];
+        m = (m > own) ? m : own;
         m_mine[it] = m;
       }
       if (carry) {
 #pragma unroll
-        for (int b = 1; b < CB; ++b)
-          if (b > wave && b < nb) m = (m > bmr[b]) ? m : bmr[b];
+        for (int b = 0; b < CB; ++b) m = (m > bmr[b]) ? m : bmr[b];
         m_run[it] = m;
       }
     }
@@ -547,12 +602,15 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
 #pragma unroll
       for (int it = 0; it < 2; ++it) {
         if (it == 1 || wave < nbA) {
-          const float corr = exp_f32_le0_tab(__fsub_rn(m_prev[it], m_mine[it]), L.etab);
+          // (exp(0) = 1 where no row's running maximum moves)
+          float corr = 1.0f;
+          if (__builtin_amdgcn_ballot_w64(m_prev[it] != m_mine[it]) != 0)
+            corr = exp_f32_le0_fast(__fsub_rn(m_prev[it], m_mine[it]), L.etab);
           float p[2][4];
 #pragma unroll
           for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p[kt][i] = exp_f32_le0_tab(__fsub_rn(s[it][kt][i], m_mine[it]), L.etab);
+            for (int i = 0; i < 4; ++i) p[kt][i] = exp_f32_le0_fast(__fsub_rn(s[it][kt][i], m_mine[it]), L.etab);
           // tree_sum over the 32 keys (key = 16 kt + 4 lg + i): bits 0-1 in
           // registers, bit 2 = lane bit 4, bit 3 = lane bit 5, bit 4 = kt
           float t[2];
@@ -567,26 +625,48 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
             t[kt] = __fadd_rn(__uint_as_float(q.a), __uint_as_float(q.b));
           }
           const float psum = __fadd_rn(t[0], t[1]);
-          // pv = P * vs (keys past kv_len: vs taken as 0, P is 0 there)
-          float pmx = 0.0f;
+          // pv = P * vs
+          float pmx = 0.0f, pmn = 0.0f;
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt) {
-            const float vv[4] = {vsr[kt][0], vsr[kt][1], vsr[kt][2], vsr[kt][3]};
+          for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const int key = j * KB + 16 * kt + 4 * lg + i;
-              p[kt][i] = __fmul_rn(p[kt][i], key < kv_len ? vv[i] : 0.0f);
+              p[kt][i] = __fmul_rn(p[kt][i], vsr[kt][i]);
               pmx = fmaxf(pmx, p[kt][i]);
+              pmn = fminf(pmn, p[kt][i]);
             }
-          }
           LanePair pr = lane_pair16(__float_as_uint(pmx));
           pmx = fmaxf(__uint_as_float(pr.a), __uint_as_float(pr.b));
           pr = lane_pair32(__float_as_uint(pmx));
           pmx = fmaxf(__uint_as_float(pr.a), __uint_as_float(pr.b));
           const float pmax = __fmul_rn(pmx, inv127());
-          const double y = rcp64(pmax);
+          // P8 = rint(RN(pv / pmax)): t = pv * r + 1.5 * 2^23 holds rint(pv * r) in
+          // its low bits, r = rcp(pmax) within 1 ulp, so pv * r is within
+          // 127 * 2^-22 of the quotient (0 <= quotient <= 127 (1 + 2^-23)) and
+          // the integer is the quotient's wherever pv * r lies more than
+          // 2^-14 from a half-integer.  A wave with a lane closer than that
+          // (~6 % of blocks), a pmax outside the range where r is normal, or a
+          // pv below -128 pmax (a negative scale) takes the exact quotients.
+          const float r = __builtin_amdgcn_rcpf(pmax);
+          uint32_t t8[2][4];
+          float far = 0.0f;
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float q = __fmul_rn(p[kt][i], r);
+              const float u = __fadd_rn(q, 0x1.8p+23f);
+              t8[kt][i] = __float_as_uint(u);
+              far = fmaxf(far, fabsf(__fsub_rn(q, __fsub_rn(u, 0x1.8p+23f))));
+            }
           uint32_t w8[2];
-          if (__builtin_amdgcn_ballot_w64(!(pmax >= 1.17549435e-38f)) == 0) {
+          const bool good = far < 0.5f - 0x1p-14f && pmax >= 0x1p-100f && pmax <= 0x1p+100f && pmn * r >= -128.0f;
+          if (__builtin_amdgcn_ballot_w64(!good) == 0) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+              w8[kt] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t8[kt][3], t8[kt][2], 0x0c0c0400u),
+                                             __builtin_amdgcn_perm(t8[kt][1], t8[kt][0], 0x0c0c0400u), 0x05040100u);
+          } else if (const double y = rcp64(pmax); __builtin_amdgcn_ballot_w64(!(pmax >= 1.17549435e-38f)) == 0) {
             // every row's pmax is normal: x / pmax <= 127 * (1 + 2^-23) for
             // x <= absmax, so rne alone lands in [0, 127]
 #pragma unroll
@@ -613,12 +693,6 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
         __builtin_amdgcn_sched_barrier(0);  // one unit at a time: bounds the live exp chains
       }
     }
-    // K rows, Q rows and ks | vs of chunk g + 1 (their registers were last
-    // read above)
-    load_k(g + 1, page);
-    load_q(g + 1);
-    load_sc(g + 1, page);
-    page = page_of(g + 2);
     lds_barrier();  // B2(g)
   }
 }

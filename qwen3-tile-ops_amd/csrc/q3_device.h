@@ -227,6 +227,28 @@ __device__ __forceinline__ float exp_f32_le0_tab(float x, const uint64_t *tab) {
   return (x2 <= -150.0f) ? 0.0f : y;
 }
 
+// exp_f32_le0_tab with fewer f64 operations, for throughput-bound softmax
+// loops (x <= 0, -inf or NaN).  The reduction in f32: x2 + 1.5 * 2^18 rounds x2 to
+// a multiple of 1/32 as glibc's f64 x2 + 1.5 * 2^47 does (|x2| < 2^17), and
+// r = x2 - k/32 is exact in f32.  x2 is first raised to -151: 2^-151 and all below
+// round to +0, glibc's result for x2 <= -150 (2^-150 is the tie that goes to
+// +0); the IEEE maximum keeps a NaN.  Equal to exp_f32_le0_tab on every float.
+__device__ __forceinline__ float exp_f32_le0_fast(float x, const uint64_t *tab) {
+  const float x2 = __builtin_elementwise_maximum(__fmul_rn(x, bits_f32(0x3FB8AA3Bu)), -151.0f);
+  const float shift = 0x1.8p+18f;
+  const float kf = __fadd_rn(x2, shift);
+  const uint32_t ki = f32_bits(kf);
+  const double r = static_cast<double>(__fsub_rn(x2, __fsub_rn(kf, shift)));
+  uint64_t t = tab[ki & 31u];
+  t += static_cast<uint64_t>(ki << 15) << 32;
+  const double s = __longlong_as_double(static_cast<long long>(t));
+  const double z = __fma_rn(0x1.c6af84b912394p-5, r, 0x1.ebfce50fac4f3p-3);
+  const double r2 = __dmul_rn(r, r);
+  double y = __fma_rn(0x1.62e42ff0c52d6p-1, r, 1.0);
+  y = __fma_rn(z, r2, y);
+  return __double2float_rn(__dmul_rn(y, s));
+}
+
 __device__ __forceinline__ float inv127() { return 1.0f / 127.0f; }
 
 // ref_qwen3.py:69-76: one element of aquant with an external scale.
