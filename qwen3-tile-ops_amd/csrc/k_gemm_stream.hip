@@ -154,32 +154,35 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
     }
   }
   constexpr bool HEADS = EPI == EPI_HEADQ || EPI == EPI_NRQ || EPI == EPI_QKV;
-  constexpr int RPW = (BM + NW - 1) / NW;  // head epilogue rows per wave
+  // head epilogue: 16 lanes a row, four rows per wave at a time (head_row16)
+  constexpr int HR = HEADS ? BM / (4 * NW) : 1;
+  static_assert(!HEADS || BM % (4 * NW) == 0, "whole waves of head rows");
   // loads that depend on another global load (device-side positions, per-row
   // tables) wait for the epilogue; only independent ones are issued here
   const bool pre_cs = do_norm && !a.cs_row_pos && !a.cs_row_dev;
   const bool pre_pg = qd.table && !qd.pos_dev && !qd.row_pos;
-  float hw0 = 0.0f, hw1 = 0.0f, hcr[RPW], hsr[RPW];
-  // pre_pg: lane q < RPW holds the page id of the wave's row q (a per-lane
-  // value, so nothing waits for it before the epilogue reads it)
-  uint32_t hpg = 0;
+  const bool cs_vec = ((reinterpret_cast<uintptr_t>(a.cos_t) | reinterpret_cast<uintptr_t>(a.sin_t) |
+                        static_cast<uintptr_t>(4 * a.ld_cs)) & 15) == 0;
+  const int hq = lane & 15;
+  auto head_row = [&](int i) { return 4 * (wave + NW * i) + (lane >> 4); };  // the lane's row of round i
+  HeadOps ho[HR];
+  uint32_t hpg[HR];  // its page id
   if constexpr (HEADS) {
     if (do_norm) {
-      hw0 = nw[static_cast<int64_t>(lane) * a.nw_stride];
-      hw1 = nw[static_cast<int64_t>(lane + 64) * a.nw_stride];
+      const bool nw_vec = a.nw_stride == 1 && (reinterpret_cast<uintptr_t>(nw) & 15) == 0;
+      load4(nw + 4 * hq * a.nw_stride, a.nw_stride, nw_vec, ho[0].w);
+      load4(nw + (64 + 4 * hq) * a.nw_stride, a.nw_stride, nw_vec, ho[0].w + 4);
     }
 #pragma unroll
-    for (int q = 0; q < RPW; ++q) {
-      const int mm = min(m0 + min(wave + NW * q, BM - 1), M - 1);
-      hcr[q] = hsr[q] = 0.0f;
+    for (int i = 0; i < HR; ++i) {
+      const int mm = min(m0 + head_row(i), M - 1);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ho[i].w[e] = ho[0].w[e];
       if (pre_cs) {
-        hcr[q] = a.cos_t[static_cast<int64_t>(mm) * a.ld_cs + lane];
-        hsr[q] = a.sin_t[static_cast<int64_t>(mm) * a.ld_cs + lane];
+        load4(a.cos_t + static_cast<int64_t>(mm) * a.ld_cs + 4 * hq, 1, cs_vec, ho[i].c);
+        load4(a.sin_t + static_cast<int64_t>(mm) * a.ld_cs + 4 * hq, 1, cs_vec, ho[i].s);
       }
-    }
-    if (pre_pg && lane < RPW) {
-      const int mm = min(m0 + min(wave + NW * lane, BM - 1), M - 1);
-      hpg = qd.table[(qd.pos0 + static_cast<uint32_t>(mm)) / qd.page_tokens];
+      if (pre_pg) hpg[i] = qd.table[(qd.pos0 + static_cast<uint32_t>(mm)) / qd.page_tokens];
     }
   }
 
@@ -424,76 +427,75 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
   } else {
     // f32 tile through LDS so that a wave can walk whole rows
     __syncthreads();
+    if constexpr (EPI == EPI_SWIGLUQ) {
+      float gv[MT * NT * 4], uv[MT * NT * 4], sv[MT * NT * 4];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            gv[(mt * NT + nt) * 4 + i] = acc[0][mt][nt][i];
+            uv[(mt * NT + nt) * 4 + i] = acc[NMAT - 1][mt][nt][i];
+          }
+      swiglu_n(gv, uv, sv, tab);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[0][mt][nt][i] = sv[(mt * NT + nt) * 4 + i];
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          float v = acc[0][mt][nt][i];
-          if constexpr (EPI == EPI_SWIGLUQ) v = swiglu_tab(acc[0][mt][nt][i], acc[NMAT - 1][mt][nt][i], tab);
-          tile[(mt * 16 + lg * 4 + i) * S::LDT + wn * S::WN + nt * 16 + lr] = v;
-        }
+        for (int nt = 0; nt < NT; ++nt)
+          tile[(mt * 16 + lg * 4 + i) * S::LDT + wn * S::WN + nt * 16 + lr] = acc[0][mt][nt][i];
     __syncthreads();
-    if constexpr (EPI == EPI_HEADQ || EPI == EPI_NRQ || EPI == EPI_QKV) {
-      // group_gemm.h:173-193 / norm_rope_quant.h:17-86 per (row, head), on
-      // the operands loaded at the start (step 0) where they were independent
-      // of other loads; rows past M store nothing
+    if constexpr (HEADS) {
+      // on the operands loaded at the start (step 0) where they were
+      // independent of other loads; rows past M store nothing
       static_assert(S::BN == 128, "one head (128 columns) per tile");
 #pragma unroll
-      for (int q = 0; q < RPW; ++q) {
-        const int rr = min(wave + NW * q, BM - 1);
-        const bool store = wave + NW * q < BM && m0 + rr < M;
+      for (int i = 0; i < HR; ++i) {
+        const int rr = head_row(i);
+        const bool store = m0 + rr < M;
         const int mm = min(m0 + rr, M - 1);
         int8_t *row8;
         float *sp;
         if (pre_pg)
-          qdest_slot(qd, __builtin_amdgcn_readlane(hpg, q), qd.pos0 + static_cast<uint32_t>(mm), nb / 128, &row8,
-                     &sp);
+          qdest_slot(qd, hpg[i], qd.pos0 + static_cast<uint32_t>(mm), nb / 128, &row8, &sp);
         else
           qdest_row(qd, mm, nb / 128, &row8, &sp);
         if (do_norm && !pre_cs) {
           const int64_t crow = a.cs_row_pos ? static_cast<int64_t>(a.cs_row_pos[mm])
                                             : mm + static_cast<int64_t>(a.cs_row_dev ? *a.cs_row_dev : 0);
-          hcr[q] = a.cos_t[crow * a.ld_cs + lane];
-          hsr[q] = a.sin_t[crow * a.ld_cs + lane];
+          load4(a.cos_t + crow * a.ld_cs + 4 * hq, 1, cs_vec, ho[i].c);
+          load4(a.sin_t + crow * a.ld_cs + 4 * hq, 1, cs_vec, ho[i].s);
         }
-        float t0 = tile[rr * S::LDT + lane];
-        float t1 = tile[rr * S::LDT + lane + 64];
-        if (do_norm) head_norm_rope_regs(t0, t1, hw0, hw1, hcr[q], hsr[q], a.inv_hd, true);
-        const float mx = max64(fmaxf(fabsf(t0), fabsf(t1)));
-        const float scale = __fmul_rn(mx, inv127());
-        const double y = rcp64(scale);
-        const int8_t q0 = static_cast<int8_t>(quant_rcp(t0, y));
-        const int8_t q1 = static_cast<int8_t>(quant_rcp(t1, y));
+        float t[8], scale;
+        uint32_t q8[2];
+        load4(tile + rr * S::LDT + 4 * hq, 1, true, t);
+        load4(tile + rr * S::LDT + 64 + 4 * hq, 1, true, t + 4);
+        head_row16(t, do_norm, ho[i], a.inv_hd, &scale, q8);
         if (store) {
-          row8[lane] = q0;
-          row8[lane + 64] = q1;
-          if (lane == 0) *sp = scale;
+          store4(row8 + 4 * hq, q8[0]);
+          store4(row8 + 64 + 4 * hq, q8[1]);
+          if (hq == 0) *sp = scale;
         }
       }
     } else if constexpr (EPI == EPI_SWIGLUQ) {
-      // swiglu_quant.h:195-231: per 256-column group absmax * (1/127)
       static_assert(S::BN % 256 == 0, "whole quantisation groups");
-      for (int rr = wave; rr < BM; rr += NW) {
+      for (int r0 = 4 * wave; r0 < BM; r0 += 4 * NW) {
+        const int rr = r0 + (lane >> 4);
         const int m = m0 + rr;
-        if (m >= M) break;
 #pragma unroll
-        for (int q = 0; q < S::BN / 256; ++q) {
-          float v[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = tile[rr * S::LDT + q * 256 + lane + 64 * j];
-          float mx = 0.0f;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fabsf(v[j]));
-          mx = max64(mx);
-          const float scale = __fmul_rn(mx, inv127());
-          const double y = rcp64(scale);
-          int8_t *dst = a.s8 + static_cast<int64_t>(m) * a.lds8 + n0 + q * 256;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dst[lane + 64 * j] = static_cast<int8_t>(quant_rcp(v[j], y));
-          if (lane == 0) a.ss[static_cast<int64_t>(m) * a.ldss + ((n0 + q * 256) / 256) * a.ss_col] = scale;
-        }
+        for (int q = 0; q < S::BN / 256; ++q)
+          quant256_row16(tile + rr * S::LDT + q * 256, lane & 15, m < M,
+                         a.s8 + static_cast<int64_t>(m) * a.lds8 + n0 + q * 256,
+                         a.ss + static_cast<int64_t>(m) * a.ldss + ((n0 + q * 256) / 256) * a.ss_col);
       }
     }
   }

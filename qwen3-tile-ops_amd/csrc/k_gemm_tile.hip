@@ -333,65 +333,78 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
   } else {
     // f32 tile through LDS (the stages are free now) so a wave can walk rows
     float *tile = reinterpret_cast<float *>(smem);
+    if constexpr (EPI == EPI_SWIGLUQ) {
+      float gv[MT * NT * 4], uv[MT * NT * 4], sv[MT * NT * 4];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            gv[(mt * NT + nt) * 4 + i] = acc[0][mt][nt][i];
+            uv[(mt * NT + nt) * 4 + i] = acc[NMAT - 1][mt][nt][i];
+          }
+      swiglu_n(gv, uv, sv, tab);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[0][mt][nt][i] = sv[(mt * NT + nt) * 4 + i];
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          float v = acc[0][mt][nt][i];
-          if constexpr (EPI == EPI_SWIGLUQ) v = swiglu_tab(acc[0][mt][nt][i], acc[NMAT - 1][mt][nt][i], tab);
-          tile[(wm * S::WM + mt * 16 + lg * 4 + i) * S::LDT + wn * S::WN + nt * 16 + lr] = v;
-        }
+        for (int nt = 0; nt < NT; ++nt)
+          tile[(wm * S::WM + mt * 16 + lg * 4 + i) * S::LDT + wn * S::WN + nt * 16 + lr] = acc[0][mt][nt][i];
     __syncthreads();
     if constexpr (EPI == EPI_HEADQ || EPI == EPI_NRQ || EPI == EPI_QKV) {
-      // group_gemm.h:173-193 / norm_rope_quant.h:17-86 per (row, head).
-      // Pass 1 loads every operand of the wave's rows (gains, cos/sin rows,
-      // destination slots through the page table) as independent loads
-      // issued together; pass 2 computes and stores.  Walking rows with
-      // their loads inside would wait for a chain of dependent loads per
-      // row.  Rows past M load row M - 1's operands and store nothing.
-      static_assert(BN == 128, "one head (128 columns) per tile");
-      constexpr int RPW = (BM + S::NW - 1) / S::NW;  // rows per wave
-      float w0 = 0.0f, w1 = 0.0f, cr[RPW], sr[RPW];
-      int8_t *row8[RPW];
-      float *sp[RPW];
-      int64_t cs_off = 0;
+      // group_gemm.h:173-193 / norm_rope_quant.h:17-86 per (row, head), 16
+      // lanes a row, four rows per wave (head_row16).  Every operand is
+      // loaded (gains, cos/sin rows, destination slots through the page
+      // table) before the first is used.  Rows past M load row M - 1's
+      // operands and store nothing.
+      static_assert(BN == 128 && BM == 4 * S::NW, "one head (128 columns) and four rows per wave");
+      const int hq = lane & 15;
+      const int rr = 4 * wave + (lane >> 4);
+      const int mm = min(m0 + rr, M - 1);
+      HeadOps ho;
       if (do_norm) {
-        w0 = nw[static_cast<int64_t>(lane) * a.nw_stride];
-        w1 = nw[static_cast<int64_t>(lane + 64) * a.nw_stride];
-        if (a.cs_row_dev) cs_off = *a.cs_row_dev;
+        const bool nw_vec = a.nw_stride == 1 && (reinterpret_cast<uintptr_t>(nw) & 15) == 0;
+        load4(nw + 4 * hq * a.nw_stride, a.nw_stride, nw_vec, ho.w);
+        load4(nw + (64 + 4 * hq) * a.nw_stride, a.nw_stride, nw_vec, ho.w + 4);
+        const bool cs_vec = ((reinterpret_cast<uintptr_t>(a.cos_t) | reinterpret_cast<uintptr_t>(a.sin_t) |
+                              static_cast<uintptr_t>(4 * a.ld_cs)) & 15) == 0;
+        const int64_t crow = a.cs_row_pos ? static_cast<int64_t>(a.cs_row_pos[mm])
+                                          : mm + static_cast<int64_t>(a.cs_row_dev ? *a.cs_row_dev : 0);
+        load4(a.cos_t + crow * a.ld_cs + 4 * hq, 1, cs_vec, ho.c);
+        load4(a.sin_t + crow * a.ld_cs + 4 * hq, 1, cs_vec, ho.s);
       }
-#pragma unroll
-      for (int q = 0; q < RPW; ++q) {
-        const int mm = min(m0 + min(wave + S::NW * q, BM - 1), M - 1);
-        cr[q] = sr[q] = 0.0f;
-        if (do_norm) {
-          const int64_t crow = a.cs_row_pos ? static_cast<int64_t>(a.cs_row_pos[mm]) : mm + cs_off;
-          cr[q] = a.cos_t[crow * a.ld_cs + lane];
-          sr[q] = a.sin_t[crow * a.ld_cs + lane];
-        }
-        qdest_row(qd, mm, nb / 128, &row8[q], &sp[q]);
+      int8_t *row8;
+      float *sp;
+      qdest_row(qd, mm, nb / 128, &row8, &sp);
+      float t[8], scale;
+      uint32_t q8[2];
+      load4(tile + rr * S::LDT + 4 * hq, 1, true, t);
+      load4(tile + rr * S::LDT + 64 + 4 * hq, 1, true, t + 4);
+      head_row16(t, do_norm, ho, a.inv_hd, &scale, q8);
+      if (m0 + rr < M) {
+        store4(row8 + 4 * hq, q8[0]);
+        store4(row8 + 64 + 4 * hq, q8[1]);
+        if (hq == 0) *sp = scale;
       }
-      // every row is computed (a row past M holds zeros: finite, unused)
-      // and only the stores are predicated, so the rows' independent
-      // reduction chains can interleave
+    } else if constexpr (EPI == EPI_SWIGLUQ) {
+      static_assert(BN % 256 == 0 && BM % (4 * S::NW) == 0, "whole quantisation groups, four rows per wave");
+      for (int r0 = 4 * wave; r0 < BM; r0 += 4 * S::NW) {
+        const int rr = r0 + (lane >> 4);
+        const int m = m0 + rr;
 #pragma unroll
-      for (int q = 0; q < RPW; ++q) {
-        const int rr = min(wave + S::NW * q, BM - 1);
-        const bool store = wave + S::NW * q < BM && m0 + rr < M;
-        float t0 = tile[rr * S::LDT + lane];
-        float t1 = tile[rr * S::LDT + lane + 64];
-        if (do_norm) head_norm_rope_regs(t0, t1, w0, w1, cr[q], sr[q], a.inv_hd, true);
-        const float mx = max64(fmaxf(fabsf(t0), fabsf(t1)));
-        const float scale = __fmul_rn(mx, inv127());
-        const int8_t q0 = static_cast<int8_t>(quant1(t0, scale));
-        const int8_t q1 = static_cast<int8_t>(quant1(t1, scale));
-        if (store) {
-          row8[q][lane] = q0;
-          row8[q][lane + 64] = q1;
-          if (lane == 0) *sp[q] = scale;
-        }
+        for (int q = 0; q < BN / 256; ++q)
+          quant256_row16(tile + rr * S::LDT + q * 256, lane & 15, m < M,
+                         a.s8 + static_cast<int64_t>(m) * a.lds8 + n0 + q * 256,
+                         a.ss + static_cast<int64_t>(m) * a.ldss + ((n0 + q * 256) / 256) * a.ss_col);
       }
     } else {
     for (int rr = wave; rr < BM; rr += S::NW) {
@@ -415,27 +428,9 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
           best = o > best ? o : best;
         }
         if (lane == 0) a.keys[static_cast<int64_t>(m) * a.keys_ld + blockIdx.x] = best;
-      } else if constexpr (EPI == EPI_SWIGLUQ) {
-        // swiglu_quant.h:195-231: per 256-column group absmax * (1/127)
-        static_assert(EPI != EPI_SWIGLUQ || BN % 256 == 0, "whole quantisation groups");
-#pragma unroll
-        for (int q = 0; q < BN / 256; ++q) {
-          float v[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = tile[rr * S::LDT + q * 256 + lane + 64 * j];
-          float mx = 0.0f;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fabsf(v[j]));
-          mx = max64(mx);
-          const float scale = __fmul_rn(mx, inv127());
-          int8_t *dst = a.s8 + static_cast<int64_t>(m) * a.lds8 + n0 + q * 256;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dst[lane + 64 * j] = static_cast<int8_t>(quant1(v[j], scale));
-          if (lane == 0) a.ss[static_cast<int64_t>(m) * a.ldss + ((n0 + q * 256) / 256) * a.ss_col] = scale;
-        }
       }
     }
-    }  // EPI_ARGMAX / EPI_SWIGLUQ
+    }  // EPI_ARGMAX
   }
 }
 

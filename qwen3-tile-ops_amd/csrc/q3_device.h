@@ -227,14 +227,13 @@ __device__ __forceinline__ float exp_f32_le0_tab(float x, const uint64_t *tab) {
   return (x2 <= -150.0f) ? 0.0f : y;
 }
 
-// exp_f32_le0_tab with fewer f64 operations, for throughput-bound softmax
-// loops (x <= 0, -inf or NaN).  The reduction in f32: x2 + 1.5 * 2^18 rounds x2 to
+// exp2f's main path with fewer f64 operations, for throughput-bound loops
+// (-151 <= x2 <= 200 or NaN).  The reduction in f32: x2 + 1.5 * 2^18 rounds x2 to
 // a multiple of 1/32 as glibc's f64 x2 + 1.5 * 2^47 does (|x2| < 2^17), and
-// r = x2 - k/32 is exact in f32.  x2 is first raised to -151: 2^-151 and all below
-// round to +0, glibc's result for x2 <= -150 (2^-150 is the tie that goes to
-// +0); the IEEE maximum keeps a NaN.  Equal to exp_f32_le0_tab on every float.
-__device__ __forceinline__ float exp_f32_le0_fast(float x, const uint64_t *tab) {
-  const float x2 = __builtin_elementwise_maximum(__fmul_rn(x, bits_f32(0x3FB8AA3Bu)), -151.0f);
+// r = x2 - k/32 is exact in f32.  Equal to glibc's exp2f on every float of the
+// range (checked exhaustively): 2^-150 and below round to +0, 2^128 and above
+// to +inf.
+__device__ __forceinline__ float exp2f_fast(float x2, const uint64_t *tab) {
   const float shift = 0x1.8p+18f;
   const float kf = __fadd_rn(x2, shift);
   const uint32_t ki = f32_bits(kf);
@@ -247,6 +246,19 @@ __device__ __forceinline__ float exp_f32_le0_fast(float x, const uint64_t *tab) 
   double y = __fma_rn(0x1.62e42ff0c52d6p-1, r, 1.0);
   y = __fma_rn(z, r2, y);
   return __double2float_rn(__dmul_rn(y, s));
+}
+
+// exp_f32_le0_tab (x <= 0, -inf or NaN) on exp2f_fast; the IEEE maximum
+// keeps a NaN.
+__device__ __forceinline__ float exp_f32_le0_fast(float x, const uint64_t *tab) {
+  return exp2f_fast(__builtin_elementwise_maximum(__fmul_rn(x, bits_f32(0x3FB8AA3Bu)), -151.0f), tab);
+}
+
+// RN(1 / d) for 1 <= d < 2^126: v_rcp_f32 and one Newton step, equal to the
+// IEEE quotient for all 2^23 significands (checked exhaustively on gfx950).
+__device__ __forceinline__ float rcp_ge1(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
 }
 
 __device__ __forceinline__ float inv127() { return 1.0f / 127.0f; }
@@ -365,6 +377,12 @@ __device__ __forceinline__ float lane_bcast(float x) {
 // Value of lane l (wave-uniform, a runtime value) in every lane.
 __device__ __forceinline__ float lane_read(float x, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
+// Value of lane L of each row of 16 lanes (DPP row_newbcast).
+template <int L>
+__device__ __forceinline__ float row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x150 + L, 0xf, 0xf, true));
 }
 
 // ---- wave reductions --------------------------------------------------

@@ -1,0 +1,70 @@
+"""The GEMMs' row epilogues (16 lanes a row): destinations, gains and RoPE rows
+of any alignment and stride, and SwiGLU arguments on both sides of its fast
+reciprocal's range, against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import bits_equal, describe_diff
+from test_gpu_ops import dev, host, nrq_ref, rand_gemm
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from q3ops import ops  # noqa: E402
+
+F = np.float32
+
+
+@pytest.mark.parametrize("M", [66, 130, 512])
+@pytest.mark.parametrize("off", [0, 1, 2])
+@pytest.mark.parametrize("tile", [False, True])
+def test_head_rows_any_alignment(cuda, monkeypatch, M, off, tile):
+    if tile:
+        monkeypatch.setenv("Q3_PREFILL_GEMM", "tile")
+    rng = np.random.default_rng(M + off)
+    K, N, H = 1024, 256, 2
+    a, as_, b, bs = rand_gemm(rng, M, K, N, 256)
+    nw = (1 + 0.1 * rng.normal(size=128)).astype(F)
+    ang = rng.uniform(0, 6, (M, 64))
+    cos, sin = np.cos(ang).astype(F), np.sin(ang).astype(F)
+    q8 = torch.zeros((M, N + 5), dtype=torch.int8, device=cuda)[:, off:off + N]
+    qs = torch.zeros((M, H + 1), dtype=torch.float32, device=cuda)[:, :H]
+    tnw = torch.zeros((128, 3), dtype=torch.float32, device=cuda)[:, :1]
+    tnw.copy_(dev(nw[:, None]))
+    tc, ts = (torch.zeros((M, 64 + off), dtype=torch.float32, device=cuda)[:, off:] for _ in range(2))
+    tc.copy_(dev(cos))
+    ts.copy_(dev(sin))
+    inv = F(1 / 128)
+    ref = oracle.gemm_nt_group(a, as_, b, bs, 256)
+    ops.gemm_nt_group_store(dev(a), dev(as_), dev(b), dev(bs), None, 256, q8=q8, qs=qs, nw=tnw, cos=tc, sin=ts,
+                            inv_hd=float(inv))
+    rq, rs = nrq_ref(ref, nw, cos, sin, H)
+    assert bits_equal(host(q8), rq), describe_diff(host(q8), rq)
+    assert bits_equal(host(qs), rs), describe_diff(host(qs), rs)
+    ops.gemm_nt_group_store(dev(a), dev(as_), dev(b), dev(bs), None, 256, q8=q8, qs=qs)
+    rq, rs = oracle.quant_rows_heads(ref, 128)
+    assert bits_equal(host(q8), rq) and bits_equal(host(qs), rs)
+
+
+@pytest.mark.parametrize("M", [66, 300])
+@pytest.mark.parametrize("off", [0, 3])
+@pytest.mark.parametrize("scale", [1e-4, 3e-3, 0.3])
+def test_gate_up_rows_and_range(cuda, M, off, scale):
+    """scale 0.3 gives gates of a few hundred: exp(-g) + 1 reaches 2^126 and
+    +inf, and 0 + 1."""
+    rng = np.random.default_rng(M)
+    a, as_, wg, wgs = rand_gemm(rng, M, 1024, 512, 256)
+    _, _, wu, wus = rand_gemm(rng, M, 1024, 512, 256)
+    as_ = (as_ * F(scale)).astype(F)
+    s8 = torch.zeros((M, 512 + 7), dtype=torch.int8, device=cuda)[:, off:off + 512]
+    ss = torch.zeros((M, 2), dtype=torch.float32, device=cuda)
+    ops.gemm_gate_up_swiglu_quant(dev(a), dev(as_), dev(wg), dev(wgs), dev(wu), dev(wus), s8, ss, 256)
+    g = oracle.gemm_nt_group(a, as_, wg, wgs, 256)
+    if scale == 0.3:
+        assert g.min() < -90 and g.max() > 90
+    r8, rs = oracle.quant_rows_heads(oracle.swiglu(g, oracle.gemm_nt_group(a, as_, wu, wus, 256)), 256)
+    assert bits_equal(host(s8), r8), describe_diff(host(s8), r8)
+    assert bits_equal(host(ss), rs), describe_diff(host(ss), rs)
