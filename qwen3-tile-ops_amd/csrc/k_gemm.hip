@@ -318,9 +318,9 @@ __global__ void __launch_bounds__(64) argmax_logits_kernel(const float *logits, 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t s) {
   if (a.M <= 0) return hipSuccess;
   if (a.bs_ld && a.epi != EPI_STORE && a.epi != EPI_ADD) return hipErrorInvalidValue;
-  // prefill shapes and batches of sequences: the LDS-staged tile kernel
-  // (ARGMAX over at most 64 rows, so that one row tile reads the weights once)
-  if (a.M > 16 && (a.epi != EPI_ARGMAX || a.M <= 64)) {
+  // prefill shapes, batches of sequences and every argmax: the LDS-staged
+  // tile kernel
+  if (a.M > 16 || a.epi == EPI_ARGMAX) {
     TileArgs t{};
     t.M = a.M;
     t.N = a.N;

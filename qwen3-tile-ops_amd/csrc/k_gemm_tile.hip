@@ -89,8 +89,17 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
   const int wn = wave / WGM;
   const int lr = lane & 15;
   const int lg = lane >> 4;
-  const int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
+  int nt_id = blockIdx.x, mt_id = blockIdx.y;
+  if constexpr (EPI == EPI_ARGMAX) {
+    // the row tiles of one weight tile run together on one XCD (workgroup
+    // i runs on XCD i % 8), so its rows come from HBM once
+    const int tm = (a.M + BM - 1) / BM, id = static_cast<int>(blockIdx.x);
+    nt_id = (id >> 3) / tm * 8 + (id & 7);
+    mt_id = (id >> 3) % tm;
+    if (nt_id * BN >= a.N) return;
+  }
+  const int m0 = mt_id * BM;
+  const int n0 = nt_id * BN;
   // the tile's column segment (EPI_QKV: Q, K or V; else the single matrix):
   // its weights, scales, first column within them, destination and norm
   const int8_t *B0 = a.b0;
@@ -406,31 +415,36 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                          a.s8 + static_cast<int64_t>(m) * a.lds8 + n0 + q * 256,
                          a.ss + static_cast<int64_t>(m) * a.ldss + ((n0 + q * 256) / 256) * a.ss_col);
       }
-    } else {
-    for (int rr = wave; rr < BM; rr += S::NW) {
-      const int m = m0 + rr;
-      if (m >= M) break;
-      if constexpr (EPI == EPI_ARGMAX) {
-        // lm_argmax.h:72-182: the row's (max, first column) over the tile's
-        // 128 columns as one 64-bit key; the finish kernel takes the max
-        // over the tiles
-        static_assert(EPI != EPI_ARGMAX || BN == 128, "one key per 128 columns");
-        const float t0 = tile[rr * S::LDT + lane];
-        const float t1 = tile[rr * S::LDT + lane + 64];
-        unsigned long long best = (static_cast<unsigned long long>(ordered_key(t0)) << 32) |
-                                  (0xFFFFFFFFu - static_cast<uint32_t>(n0 + lane));
-        const unsigned long long other = (static_cast<unsigned long long>(ordered_key(t1)) << 32) |
-                                         (0xFFFFFFFFu - static_cast<uint32_t>(n0 + lane + 64));
-        best = other > best ? other : best;
+    } else if constexpr (EPI == EPI_ARGMAX) {
+      // lm_argmax.h:72-182: the row's (max, first column) over the tile's
+      // 128 columns as one 64-bit key (16 lanes a row); the finish kernel
+      // takes the max over the tiles
+      static_assert(EPI != EPI_ARGMAX || (BN == 128 && BM % (4 * S::NW) == 0), "one key per 128 columns");
+      const int q = lane & 15;
+      for (int r0 = 4 * wave; r0 < BM; r0 += 4 * S::NW) {
+        const int rr = r0 + (lane >> 4);
+        float t[8];
+        load4(tile + rr * S::LDT + 4 * q, 1, true, t);
+        load4(tile + rr * S::LDT + 64 + 4 * q, 1, true, t + 4);
+        uint32_t top = ordered_key(t[0]);
+        int col = 4 * q;
 #pragma unroll
-        for (int sft = 1; sft < 64; sft <<= 1) {
+        for (int i = 1; i < 8; ++i) {  // ascending columns: the first of equal keys stays
+          const uint32_t k = ordered_key(t[i]);
+          const int c = (i < 4 ? 0 : 60) + 4 * q + i;
+          col = k > top ? c : col;
+          top = k > top ? k : top;
+        }
+        unsigned long long best =
+            (static_cast<unsigned long long>(top) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(n0 + col));
+#pragma unroll
+        for (int sft = 1; sft < 16; sft <<= 1) {
           const unsigned long long o = lane_xor_u64(best, sft);
           best = o > best ? o : best;
         }
-        if (lane == 0) a.keys[static_cast<int64_t>(m) * a.keys_ld + blockIdx.x] = best;
+        if (q == 0 && m0 + rr < M) a.keys[static_cast<int64_t>(m0 + rr) * a.keys_ld + n0 / 128] = best;
       }
     }
-    }  // EPI_ARGMAX
   }
 }
 
@@ -452,7 +466,8 @@ hipError_t launch_shape(const TileArgs &a, hipStream_t s) {
     if (e != hipSuccess) return e;
     attr_set = true;
   }
-  const dim3 grid(a.N / BN, (a.M + BM - 1) / BM);
+  const int tm = (a.M + BM - 1) / BM;
+  const dim3 grid = EPI == EPI_ARGMAX ? dim3((a.N / BN + 7) / 8 * 8 * tm) : dim3(a.N / BN, tm);
   Q3_LAUNCH((gemm_tile_kernel<BM, BN, WGM, NMAT, STAGES, KS, EPI, GROUP, BSG>), grid, dim3(S::NTHR), lds, s, a);
   return hipGetLastError();
 }
@@ -535,9 +550,16 @@ hipError_t launch_gemm_tile(const TileArgs &a, int epi, hipStream_t s) {
           return hipErrorInvalidValue;
       return launch_tile<32, 128, 2, 1, 3, 128, EPI_QKV>(a, s);
     case EPI_SWIGLUQ: return launch_tile<32, 256, 1, 2, 2, 128, EPI_SWIGLUQ>(a, s);
-    case EPI_ARGMAX:  // rows of a batch of sequences (M <= 64): the weights are read once
+    case EPI_ARGMAX:
       if (!a.keys || a.keys_ld < a.N / 128) return hipErrorInvalidValue;
-      return launch_tile<64, 128, 2, 1, 3, 256, EPI_ARGMAX>(a, s);
+      // 128-byte k-steps: 72 KiB (60 KiB) of LDS, two workgroups per CU, so
+      // that one tile's first copies and epilogue run beside the other's
+      // k-steps (a tile has only 8).  151936 columns, us with the finish
+      // launch: 20 rows 36.5, 64 rows 39.9, 100 rows 53, 256 rows 89 (256-byte
+      // steps, one workgroup per CU: 49, 50, 75, 129; 128-row tiles: 57, 57,
+      // 59, 104).
+      if (a.M <= 32) return launch_tile<32, 128, 2, 1, 3, 128, EPI_ARGMAX>(a, s);
+      return launch_tile<64, 128, 2, 1, 3, 128, EPI_ARGMAX>(a, s);
     default: return hipErrorInvalidValue;
   }
 }
