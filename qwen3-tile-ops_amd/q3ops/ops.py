@@ -11,36 +11,54 @@ non-zero status.  There is no fallback path: the HIP library must be built.
 from __future__ import annotations
 
 import ctypes as C
+from ctypes import byref
 
 import torch
 
 from ._lib import DT_F32, DT_I8, DT_I32, LM_ARGMAX, PagedKV, View, check, lib
 
-_DT = {torch.int8: DT_I8, torch.float32: DT_F32, torch.int32: DT_I32}
+# element size and dtype code of the view dtypes
+_DT = {torch.int8: (1, DT_I8), torch.float32: (4, DT_F32), torch.int32: (4, DT_I32)}
 
 
 def view(t: torch.Tensor | None):
-    """MatrixView of a tensor (kernels/matrix.h:27-34); None -> NULL."""
+    """MatrixView of a tensor (kernels/matrix.h:27-34); None -> NULL.
+
+    Each tensor attribute is read once: an operator makes up to a dozen views,
+    and with two reads of most attributes they were most of a small call's
+    host time (a one-row projection 11.7 us a call on the host)."""
     if t is None:
         return None
-    if t.dtype not in _DT:
+    known = _DT.get(t.dtype)
+    if known is None:
         raise TypeError(f"unsupported dtype {t.dtype}")
     if not t.is_cuda:
         raise ValueError("operator views must point at device memory")
-    es = t.element_size()
-    if t.dim() == 1:
-        if t.stride(0) != 1:
+    es, code = known
+    stride = t.stride()
+    if len(stride) == 1:
+        if stride[0] != 1:
             raise ValueError("1-D views must be contiguous")
-        return C.byref(View(t.data_ptr(), es, es, t.shape[0], 1, _DT[t.dtype]))
-    if t.dim() != 2 or t.stride(1) != 1:
+        return byref(View(t.data_ptr(), es, es, t.shape[0], 1, code))
+    if len(stride) != 2 or stride[1] != 1:
         raise ValueError("views must be 2-D with dense columns")
-    row_bytes = t.stride(0) * es if t.shape[0] > 1 else t.shape[1] * es
-    return C.byref(View(t.data_ptr(), row_bytes, es, t.shape[0], t.shape[1], _DT[t.dtype]))
+    rows, cols = t.shape
+    return byref(View(t.data_ptr(), (stride[0] if rows > 1 else cols) * es, es, rows, cols, code))
 
 
-def _stream(stream=None) -> C.c_void_p:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+def _stream(stream=None) -> int:
+    """The hipStream_t of the stream, or of the current device's current one
+    (read as the raw handle: a Stream object costs a microsecond)."""
+    if stream is not None:
+        return stream.cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _raw_stream(device: int) -> int:
+    """torch.cuda.current_stream(device).cuda_stream, without the object where
+    this torch has the raw getter."""
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return get(device) if get else torch.cuda.current_stream(device).cuda_stream
 
 
 def paged_kv(k: torch.Tensor, v: torch.Tensor, ks: torch.Tensor, vs: torch.Tensor,
