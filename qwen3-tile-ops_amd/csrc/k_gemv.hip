@@ -53,8 +53,12 @@ constexpr int kPartPro = 1, kPartEpi = 2;
 // the other scales before the weight stream (PRO_NONE, one matrix).
 // MT row tiles of 16 (MT > 1: plain A operand, rows past M computed on row
 // M - 1's data and not stored), their A fragments loaded AB tiles at a time.
-template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT>
+// RB: rows whose prologue operands are loaded and computed together
+// (pro_compute_rows; 1: one row, pro_compute_row).
+template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT,
+          int RB = 1>
 __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
+  static_assert(RB == 1 || (PRO != PRO_NONE && PART == 0 && MT == 1), "row batches: prologue rows");
   static_assert(PART == 0 || NT == 1, "partials: one item column per thread");
   static_assert(!BSG || (NMAT == 1 && PRO == PRO_NONE && PART == 0), "per-group B scales: plain GEMV");
   static_assert(MT == 1 || (PRO == PRO_NONE && PART == 0 && NT == 1), "row tiles: plain A operand");
@@ -128,7 +132,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
   const int part_floats = NMAT * ngroups * MR * PP;
   int8_t *a_lds = reinterpret_cast<int8_t *>(part + part_floats);
   float *as_lds = reinterpret_cast<float *>(a_lds + ((M * K + 15) & ~15));
-  float *blk = as_lds + M * (K / 256);
+  float *blk = as_lds + ((M * (K / 256) + 3) & ~3);
   __shared__ uint64_t exptab[32];
   constexpr int QW = GPW * KSTEPS / 4;  // 256-column groups per wave
 
@@ -139,7 +143,9 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
   // waits for those operands alone (vmcnt(#weight loads)) instead of for
   // everything.
   ProRow<QW, NPRO> r0;
-  if constexpr (PRO != PRO_NONE) pro_load_row<PRO, QW, NPRO>(a, ps, 0, r0);
+  ProRows<PRO, QW, RB> rb;
+  if constexpr (PRO != PRO_NONE && RB == 1) pro_load_row<PRO, QW, NPRO>(a, ps, 0, r0);
+  if constexpr (PRO != PRO_NONE && RB > 1) pro_load_rows<PRO, QW, RB>(a, ps, 0, M, rb);
   __builtin_amdgcn_sched_barrier(0);  // (issue order: prologue operands first)
   // EPI_ADD with partials: those of the thread's item column, before the
   // weights (the column j = it % NB is the same for every item it of the
@@ -243,7 +249,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
   // wait for one load per item (the store of an item would otherwise hold
   // back the next item's load)
   float basev[MT];
-  if constexpr (MT > 1) {
+  if constexpr (NT == 1) {
     if (sg.epi == EPI_ADD) {
 #pragma unroll
       for (int k = 0; k < MT; ++k) {
@@ -255,11 +261,14 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
   }
 
   if constexpr (PRO != PRO_NONE) {
-    pro_compute_row<PRO, QW, NPRO>(a, 0, r0, a_lds, as_lds, blk, blockIdx.x == 0);
-    for (int m = 1; m < M; ++m) {
-      ProRow<QW, 0> r;
-      pro_load_row<PRO, QW, 0>(a, ps, m, r);
-      pro_compute_row<PRO, QW, 0>(a, m, r, a_lds, as_lds, blk, blockIdx.x == 0);
+    if constexpr (RB > 1) {
+      pro_compute_rows<PRO, QW, RB>(a, 0, M, rb, a_lds, as_lds, blk, blockIdx.x == 0);
+      for (int m0 = RB; m0 < M; m0 += RB) {
+        pro_load_rows<PRO, QW, RB>(a, ps, m0, M, rb);
+        pro_compute_rows<PRO, QW, RB>(a, m0, M, rb, a_lds, as_lds, blk, blockIdx.x == 0);
+      }
+    } else {
+      pro_compute_row<PRO, QW, NPRO>(a, 0, r0, a_lds, as_lds, blk, blockIdx.x == 0);  // (one row)
     }
     const int8_t *arow = a_lds + (avalid ? lr : 0) * K + lg * 16;
 #pragma unroll
@@ -350,7 +359,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
     if (m >= M) continue;
     float *dst = sg.out + static_cast<int64_t>(row0 + m) * sg.ldo + ncol;
     if (sg.epi == EPI_ADD) {
-      float base = MT > 1 ? basev[k] : *dst;
+      float base = NT == 1 ? basev[k] : *dst;
       if constexpr (NEPI > 0) {
         float o = 0.0f;  // the O projection, partials in head order
 #pragma unroll
@@ -359,10 +368,14 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
         base = __fadd_rn(base, o);
       }
       *dst = __fadd_rn(base, out);
-    } else if (sg.epi == EPI_SWIGLU)
-      *dst = swiglu_tab(out, out2, exptab);
-    else
+    } else if (sg.epi == EPI_SWIGLU) {
+      const float gv[1] = {out}, uv[1] = {out2};
+      float sv[1];
+      swiglu_n(gv, uv, sv, exptab);
+      *dst = sv[0];
+    } else {
       *dst = out;
+    }
   }
 }
 
@@ -783,22 +796,31 @@ __global__ void __launch_bounds__(256) gemv_wr_kernel(GemvArgs a, int N) {
 // added in ascending order.  BSG: per-(row, K-group) B scales.  Bound by one
 // memory round trip: N / 4 workgroups instead of the MFMA tile kernel's
 // N / 16 (O, K = 2048 x 1024: 5.3 -> 2.7 us with cached operands).
-template <int KB, int LPG, int R, bool BSG>
+// MR > 1: 2 .. MR rows over the same weight registers, launched while the
+// 16-column tiles leave most CUs without a workgroup (up to 2048 columns).
+template <int KB, int LPG, int R, bool BSG, int MR>
 __global__ void __launch_bounds__(256) gemv_wr_plain_kernel(GemvArgs a, int N) {
   constexpr int GPJ = 64 / LPG;  // K-groups per 1024 bytes
   const int lane = threadIdx.x & 63;
   const int8_t *ap = pin_sgpr(a.a), *bp = pin_sgpr(a.seg[0].b);
   const float *asp = pin_sgpr(a.as), *bsp = pin_sgpr(a.seg[0].bs);
   float *outp = pin_sgpr(a.seg[0].out);
+  const int64_t lda = MR > 1 ? pin_sgpr(a.lda) : 0, ldas = MR > 1 ? pin_sgpr(a.ldas) : 0;
+  const int64_t ldo = MR > 1 ? pin_sgpr(a.seg[0].ldo) : 0;
   const int64_t bs_ld = BSG ? pin_sgpr(a.bs_ld) : 0;
+  const int M = MR > 1 ? a.M : 1;
   const bool add = a.seg[0].epi == EPI_ADD;
   const int row0 = (static_cast<int>(blockIdx.x) * 4 + wave_id()) * R;
-  int4 av[KB], w[R][KB];
-  float asg[KB], bsn[R][BSG ? KB : 1], base[R];
+  int4 av[MR][KB], w[R][KB];
+  float asg[MR][KB], bsn[R][BSG ? KB : 1], base[R][MR];
 #pragma unroll
-  for (int j = 0; j < KB; ++j) {
-    av[j] = *reinterpret_cast<const int4 *>(ap + 1024 * j + 16 * lane);
-    asg[j] = asp[GPJ * j + lane / LPG];
+  for (int m = 0; m < MR; ++m) {
+    const int64_t mm = MR > 1 ? min(m, M - 1) : 0;
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      av[m][j] = *reinterpret_cast<const int4 *>(ap + mm * lda + 1024 * j + 16 * lane);
+      asg[m][j] = asp[mm * ldas + GPJ * j + lane / LPG];
+    }
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -808,26 +830,30 @@ __global__ void __launch_bounds__(256) gemv_wr_plain_kernel(GemvArgs a, int N) {
       w[r][j] = *reinterpret_cast<const int4 *>(bp + static_cast<int64_t>(n) * (1024 * KB) + 1024 * j + 16 * lane);
 #pragma unroll
     for (int j = 0; j < (BSG ? KB : 1); ++j) bsn[r][j] = BSG ? bsp[n * bs_ld + GPJ * j + lane / LPG] : bsp[n];
-    base[r] = add ? outp[n] : 0.0f;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) base[r][m] = add ? outp[(MR > 1 ? min(m, M - 1) : 0) * ldo + n] : 0.0f;
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    float out = 0.0f;
 #pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      int acc = sdot4(w[r][j].x, av[j].x, 0);
-      acc = sdot4(w[r][j].y, av[j].y, acc);
-      acc = sdot4(w[r][j].z, av[j].z, acc);
-      acc = sdot4(w[r][j].w, av[j].w, acc);
-      acc += lane_xor<1>(acc);
-      acc += lane_xor<2>(acc);
-      acc += lane_xor<4>(acc);
-      if constexpr (LPG == 16) acc += lane_xor<8>(acc);
-      const float p = __fmul_rn(__fmul_rn(static_cast<float>(acc), bsn[r][BSG ? j : 0]), asg[j]);
+    for (int m = 0; m < MR; ++m) {
+      float out = 0.0f;
 #pragma unroll
-      for (int g = 0; g < GPJ; ++g) out = __fadd_rn(out, lane_read(p, g * LPG));
+      for (int j = 0; j < KB; ++j) {
+        int acc = sdot4(w[r][j].x, av[m][j].x, 0);
+        acc = sdot4(w[r][j].y, av[m][j].y, acc);
+        acc = sdot4(w[r][j].z, av[m][j].z, acc);
+        acc = sdot4(w[r][j].w, av[m][j].w, acc);
+        acc += lane_xor<1>(acc);
+        acc += lane_xor<2>(acc);
+        acc += lane_xor<4>(acc);
+        if constexpr (LPG == 16) acc += lane_xor<8>(acc);
+        const float p = __fmul_rn(__fmul_rn(static_cast<float>(acc), bsn[r][BSG ? j : 0]), asg[m][j]);
+#pragma unroll
+        for (int g = 0; g < GPJ; ++g) out = __fadd_rn(out, lane_read(p, g * LPG));
+      }
+      if (lane == 0 && row0 + r < N && m < M) outp[m * ldo + row0 + r] = add ? __fadd_rn(base[r][m], out) : out;
     }
-    if (lane == 0 && row0 + r < N) outp[row0 + r] = add ? __fadd_rn(base[r], out) : out;
   }
 }
 
@@ -898,8 +924,10 @@ __global__ void __launch_bounds__(256) qkv_heads_kernel(QkvHeadArgs a) {
   if (lane == 0) *sp = scale;
 }
 
-template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT>
+template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT,
+          int RB = 1>
 hipError_t launch_t(const GemvArgs &a, int ncols, hipStream_t s, int ry = 1) {
+  if (PRO != PRO_NONE && RB == 1 && a.M != 1) return hipErrorInvalidValue;
   constexpr int NB = 16 * NT;
   // the prologue gives each wave GPW * KSTEPS / 4 groups of 256 columns
   if (PRO != PRO_NONE && a.K != 256 * GPW * KSTEPS) return hipErrorInvalidValue;
@@ -909,7 +937,8 @@ hipError_t launch_t(const GemvArgs &a, int ncols, hipStream_t s, int ry = 1) {
   size_t lds = sizeof(float) * NMAT * ngroups * 16 * MT * (NB + 1);
   if (MT > 1) lds += sizeof(float) * 16 * MT * ngroups;  // the staged A scales
   if (PRO != PRO_NONE)
-    lds += ((a.M * a.K + 15) & ~15) + sizeof(float) * (a.M * (a.K / 256) + a.K / 32);
+    lds += ((a.M * a.K + 15) & ~15) + sizeof(float) * (((a.M * (a.K / 256) + 3) & ~3) +
+                                                       std::max(a.K / 32, pro_rows_blk<GPW * KSTEPS / 4, RB>()));
   // dynamic LDS beyond 64 KiB (row tiles) must be allowed once; the kernel's
   // static LDS (the exp table) counts against the same 160 KiB
   constexpr size_t kMaxDyn = 159 * 1024;
@@ -918,13 +947,13 @@ hipError_t launch_t(const GemvArgs &a, int ncols, hipStream_t s, int ry = 1) {
     static bool attr_set = false;
     if (!attr_set) {
       const hipError_t e = hipFuncSetAttribute(
-          reinterpret_cast<const void *>(&gemv_kernel<GPW, KSTEPS, NT, NMAT, PRO, PART, BSG, MT, AB>),
+          reinterpret_cast<const void *>(&gemv_kernel<GPW, KSTEPS, NT, NMAT, PRO, PART, BSG, MT, AB, RB>),
           hipFuncAttributeMaxDynamicSharedMemorySize, kMaxDyn);
       if (e != hipSuccess) return e;
       attr_set = true;
     }
   }
-  Q3_LAUNCH((gemv_kernel<GPW, KSTEPS, NT, NMAT, PRO, PART, BSG, MT, AB>), dim3(ncols / NB, ry), dim3(256), lds, s, a);
+  Q3_LAUNCH((gemv_kernel<GPW, KSTEPS, NT, NMAT, PRO, PART, BSG, MT, AB, RB>), dim3(ncols / NB, ry), dim3(256), lds, s, a);
   return hipGetLastError();
 }
 
@@ -959,13 +988,20 @@ hipError_t dispatch_rows(const GemvArgs &a, int ncols, hipStream_t s) {
 // The prologue kinds (a template parameter, so that no branch on a kernel
 // argument precedes the first loads) are built for K = 1024, 2048 and 3072
 // with group 256 and 16-column tiles.
-template <int NMAT, int PRO, int PART>
+template <int NMAT, int PRO, int RB>
+hipError_t dispatch_pro_rows(const GemvArgs &a, int ncols, hipStream_t s) {
+  if (a.K == 1024) return launch_t<1, 4, 1, NMAT, PRO, 0, false, 1, 1, RB>(a, ncols, s);
+  if (a.K == 2048) return launch_t<2, 4, 1, NMAT, PRO, 0, false, 1, 1, RB>(a, ncols, s);
+  if (a.K == 3072) return launch_t<3, 4, 1, NMAT, PRO, 0, false, 1, 1, RB>(a, ncols, s);
+  return hipErrorInvalidValue;
+}
+
+template <int NMAT, int PRO>
 hipError_t dispatch_pro(const GemvArgs &a, int ncols, hipStream_t s) {
   if (a.group != 256) return hipErrorInvalidValue;
-  if (a.K == 1024) return launch_t<1, 4, 1, NMAT, PRO, PART>(a, ncols, s);
-  if (a.K == 2048) return launch_t<2, 4, 1, NMAT, PRO, PART>(a, ncols, s);
-  if (a.K == 3072) return launch_t<3, 4, 1, NMAT, PRO, PART>(a, ncols, s);
-  return hipErrorInvalidValue;
+  if (a.M == 1) return dispatch_pro_rows<NMAT, PRO, 1>(a, ncols, s);
+  if (a.M > 4 && a.M <= 8) return dispatch_pro_rows<NMAT, PRO, 8>(a, ncols, s);
+  return dispatch_pro_rows<NMAT, PRO, 4>(a, ncols, s);  // (16 rows of K = 3072 and eight rows' sums exceed 64 KiB)
 }
 
 template <int NT, int NMAT>
@@ -989,9 +1025,9 @@ hipError_t dispatch_k(const GemvArgs &a, int ncols, hipStream_t s) {
     return hipErrorInvalidValue;
   }
   if constexpr (NT == 1) {
-    if (a.pro == PRO_NORM) return dispatch_pro<NMAT, PRO_NORM, 0>(a, ncols, s);
-    if (a.pro == PRO_EMBED) return dispatch_pro<NMAT, PRO_EMBED, 0>(a, ncols, s);
-    if (a.pro == PRO_QUANT) return dispatch_pro<NMAT, PRO_QUANT, 0>(a, ncols, s);
+    if (a.pro == PRO_NORM) return dispatch_pro<NMAT, PRO_NORM>(a, ncols, s);
+    if (a.pro == PRO_EMBED) return dispatch_pro<NMAT, PRO_EMBED>(a, ncols, s);
+    if (a.pro == PRO_QUANT) return dispatch_pro<NMAT, PRO_QUANT>(a, ncols, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1061,22 +1097,31 @@ int wr_rows(const GemvArgs &a, int ncols) {
   return R;
 }
 
-// One row with an int8 A row, plain or residual store, one segment: 1 weight
-// row per wave up to 2048 columns (256-512 workgroups), 2 above.
+// Up to 8 int8 A rows, plain or residual store, one segment: 1 weight row per
+// wave up to 2048 columns (256-512 workgroups); one A row also above, with 2.
+// Against the 16-column tiles, us a call in a graph: 3072 x 1024, 4 rows
+// 4.51 -> 3.00, 8 rows 4.71 -> 4.26; 2048 x 1024, 8 rows 3.94 -> 3.65;
+// 1024 x 2048, 4 rows 3.10 -> 2.81, but 5 rows 3.09 -> 3.46 (one K-step per
+// tile leaves nothing to win), so K = 1024 stops at 4 rows.
 bool wr_plain(const GemvArgs &a, int ncols) {
   const int epi = a.seg[0].epi;
-  return a.M == 1 && a.pro == PRO_NONE && a.nseg == 1 && !a.part && !a.clear && ncols < 65536 && ncols % 8 == 0 &&
-         (epi == EPI_STORE || epi == EPI_ADD) && a.K % 1024 == 0 && a.K >= 1024 && a.K <= 3072 &&
-         (a.group == 256 || (a.group == 128 && a.K <= 2048)) &&
+  return a.M <= (ncols > 2048 ? 1 : a.K > 1024 ? 8 : 4) && a.pro == PRO_NONE && a.nseg == 1 && !a.part && !a.clear && ncols < 65536 &&
+         ncols % 8 == 0 && (epi == EPI_STORE || epi == EPI_ADD) && a.K % 1024 == 0 && a.K >= 1024 && a.K <= 3072 &&
+         (a.group == 256 || (a.group == 128 && a.K <= 2048)) && (a.M == 1 || a.lda % 16 == 0) &&
          (reinterpret_cast<uintptr_t>(a.a) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.seg[0].b) & 15) == 0;
 }
 
 template <int KB, int LPG, bool BSG>
 hipError_t launch_wr_plain(const GemvArgs &a, int ncols, hipStream_t s) {
-  if (ncols <= 2048)
-    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 1, BSG>), dim3(ncols / 4), dim3(256), 0, s, a, ncols);
+  const dim3 grid(ncols / 4), block(256);
+  if (a.M > 4)
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 1, BSG, 8>), grid, block, 0, s, a, ncols);
+  else if (a.M > 1)
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 1, BSG, 4>), grid, block, 0, s, a, ncols);
+  else if (ncols <= 2048)
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 1, BSG, 1>), grid, block, 0, s, a, ncols);
   else
-    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 2, BSG>), dim3(ncols / 8), dim3(256), 0, s, a, ncols);
+    Q3_LAUNCH((gemv_wr_plain_kernel<KB, LPG, 2, BSG, 1>), dim3(ncols / 8), block, 0, s, a, ncols);
   return hipGetLastError();
 }
 

@@ -124,12 +124,11 @@ thread_local const LaunchEvents *g_launch_events = nullptr;
 namespace {
 
 constexpr uint32_t kPageTokens = 32;
-// Rows of a chunk on the GEMVs with prologues (forward_small): each workgroup
-// rebuilds the int8 rows one after the other, ~1 us per row and launch, so
-// from 5 rows on the row kernels and plain GEMVs of the 17-64-row path are
-// faster (28 layers, us: 4 rows 1130 against 1169, 5 1217 / 1166, 8 1461 /
-// 1183, 16 2170 / 1207).
-constexpr int kMaxSmallRows = 4;
+// Rows of a chunk (forward_small) or of a batch on the GEMVs with prologues,
+// which save the norm and quant launches but rebuild the int8 rows in every
+// workgroup, up to 8 rows together (28 layers, us, against the row kernels and
+// plain GEMVs: 2 rows 917 / 1050, 4 954 / 1053, 8 1134 / 1143, 9 1381 / 1173).
+constexpr int kMaxSmallRows = 8;
 
 int hip_status(hipError_t e) { return e == hipSuccess ? Q3_OK : Q3_ERR_HIP; }
 
@@ -1432,17 +1431,32 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
     r.group = 256;
     return hip_status(q3::launch_rows(r, s));
   };
-  Q3_TRY(rows(2, layer_ptrs(m, 0).n1));
   // up to 64 rows: the GEMMs run on the 16-column GEMV tiles (every CU
   // streams a slice of the weights; the rows come from L2), with the head
   // epilogues and the SwiGLU quantisation as launches of their own
   const bool gv = q3::gemv_rows_supported(M, H, 256, QW + 2 * KW) && q3::gemv_rows_supported(M, QW, HD, H) &&
                   q3::gemv_rows_supported(M, I, 256, H) && q3::gemv_rows_supported(M, H, 256, I);
+  // up to 8 rows: RMSNorm (layer 0: the embedding) and the quantisations run
+  // in the GEMVs' prologues
+  const bool pro = gv && small_path(y, n);
+  if (!pro) Q3_TRY(rows(2, layer_ptrs(m, 0).n1));
   float *qf = at<float>(m, y.kQ), *kf = at<float>(m, y.kK), *vf = at<float>(m, y.kV);
   float *swf = at<float>(m, y.kSW);
   for (uint32_t L = 0; L < y.layers; ++L) {
     const LayerPtrs lp = layer_ptrs(m, L);
-    if (L != 0) Q3_TRY(rows(1, lp.n1));
+    if (L != 0 && !pro) Q3_TRY(rows(1, lp.n1));
+    // a prologue GEMV's A operand: quant256(rmsnorm of the f32 rows src, w)
+    auto norm_pro = [&](q3::GemvArgs &g, const float *w) {
+      g.a = nullptr;
+      g.pro = q3::PRO_NORM;
+      g.x = x;
+      g.ldx = H;
+      g.w_pre = w;
+      g.inv_pre = 1.0f / static_cast<float>(H);
+      g.h_out = h;
+      g.h8_out = h8;
+      g.hs_out = hs;
+    };
     if (gv) {
       // Q | K | V rows in f32, then the head epilogues of every (row, head):
       // Q (norm, RoPE, quant) into the dense q8/qs rows, K (norm, RoPE,
@@ -1456,6 +1470,17 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.seg[0] = gemv_seg(0, QW, q3::EPI_STORE, lp.wq, lp.wqs, qf, QW);
       g.seg[1] = gemv_seg(QW, QW + KW, q3::EPI_STORE, lp.wk, lp.wks, kf, KW);
       g.seg[2] = gemv_seg(QW + KW, QW + 2 * KW, q3::EPI_STORE, lp.wv, lp.wvs, vf, KW);
+      if (pro) {
+        norm_pro(g, lp.n1);
+        if (L == 0) {
+          g.pro = q3::PRO_EMBED;
+          g.emb = at<const int8_t>(m, y.kEMB);
+          g.emb_s = at<const float>(m, y.kEMB + static_cast<int64_t>(V) * H);
+          g.ids = ids;
+          g.vocab = V;
+          g.x_out = x;
+        }
+      }
       Q3_HIP(q3::launch_gemv(g, s));
     }
     if (gv && split) {  // the head epilogues are part of the split attention
@@ -1596,7 +1621,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.ldo = H;
       Q3_HIP(q3::launch_gemm(g, s));
     }
-    Q3_TRY(rows(1, lp.n2));
+    if (!pro) Q3_TRY(rows(1, lp.n2));
     if (gv) {  // gate/up + SwiGLU (f32 rows), then the per-256-column quant
       q3::GemvArgs g = gemv_args(M, H, 256);
       g.a = h8;
@@ -1607,6 +1632,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.seg[0] = gemv_seg(0, I, q3::EPI_SWIGLU, lp.wg, lp.wgs, swf, I);
       g.seg[0].b2 = lp.wu;
       g.seg[0].bs2 = lp.wus;
+      if (pro) norm_pro(g, lp.n2);
       Q3_HIP(q3::launch_gemv(g, s));
       q3::RowArgs r{};
       r.mode = 0;
@@ -1619,7 +1645,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       r.hs = ss;
       r.ldhs = I / 256;
       r.group = 256;
-      Q3_HIP(q3::launch_rows(r, s));
+      if (!pro) Q3_HIP(q3::launch_rows(r, s));
     } else {  // gate/up + SwiGLU + quant
       q3::GateUpArgs u;
       std::memset(&u, 0, sizeof(u));
@@ -1652,6 +1678,14 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.ldas = I / 256;
       g.nseg = 1;
       g.seg[0] = gemv_seg(0, H, q3::EPI_ADD, lp.wd, lp.wds, x, H);
+      if (pro) {  // quant256 of the SwiGLU rows
+        g.a = nullptr;
+        g.pro = q3::PRO_QUANT;
+        g.x = swf;
+        g.ldx = I;
+        g.h8_out = s8;
+        g.hs_out = ss;
+      }
       Q3_HIP(q3::launch_gemv(g, s));
     } else {
       q3::GemmArgs g = gemm_args(M, H, I, 256, s8, ss, lp.wd, lp.wds);

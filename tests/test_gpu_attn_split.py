@@ -119,3 +119,28 @@ def test_one_row_whole_row_gemm(cuda, K, group, N, per_group):
     xt = dev(x)
     ops.gemm_nt_group_store(dev(a), dev(as_), dev(b), dev(bs), None, group, add=xt)
     assert bits_equal(host(xt), (ref + x).astype(np.float32))
+
+
+@pytest.mark.parametrize("M", [2, 4, 5, 8])
+@pytest.mark.parametrize("K,group", [(1024, 128), (1024, 256), (2048, 128), (2048, 256), (3072, 256)])
+@pytest.mark.parametrize("per_group", [False, True])
+def test_few_rows_whole_row_gemm(cuda, M, K, group, per_group):
+    """2 to 8 rows over the same weight registers, strided operands."""
+    rng = np.random.default_rng(K + M + group)
+    N = 384
+    a, as_, b, bs = rand_gemm(rng, M, K, N, group)
+    if per_group:
+        bs = rng.uniform(1e-3, 1e-1, (N, K // group)).astype(np.float32)
+    ta = torch.zeros((M, K + 16), dtype=torch.int8, device=cuda)[:, :K]
+    ta.copy_(dev(a))
+    tas = torch.zeros((M, K // group + 1), device=cuda)[:, :K // group]
+    tas.copy_(dev(as_))
+    ref = (oracle.gemm_nt_group_bg if per_group else oracle.gemm_nt_group)(a, as_, b, bs, group)
+    out = torch.zeros((M + 1, N + 3), dtype=torch.float32, device=cuda)
+    ops.gemm_nt_group_store(ta, tas, dev(b), dev(bs), out[:M, :N], group)
+    assert bits_equal(host(out[:M, :N]), ref), describe_diff(host(out[:M, :N]), ref)
+    assert not out[M].any() and not out[:, N:].any()
+    x = rng.normal(size=(M, N)).astype(np.float32)
+    xt = dev(x)
+    ops.gemm_nt_group_store(ta, tas, dev(b), dev(bs), None, group, add=xt)
+    assert bits_equal(host(xt), (ref + x).astype(np.float32))
