@@ -22,10 +22,19 @@
 // flight (128 KiB for gate/up), enough to cover last-level-cache latency.
 //
 // Per-group dequantisation: 4 VALU operations per output element and group
-// (cvt, two RN multiplies, add).  The int32 group sums are double buffered by
-// group parity: group g is dequantised right after the first MFMAs of group
-// g + 1 are issued, so the VALU work of one group overlaps the MFMAs of the
-// next.
+// (cvt, two RN multiplies, add).  With CB = 2 the int32 group sums are double
+// buffered by group parity: group g is dequantised right after the first MFMAs
+// of group g + 1 are issued, so the VALU work of one group overlaps the MFMAs
+// of the next.  CB = 1: one buffer, dequantised after the group's last slice
+// (half the registers; the other waves of the SIMD fill the gap).
+//
+// What bounds it: operand bytes per MFMA (16 cycles).  A wave reads 1 KiB of A
+// from LDS per NT * NMAT of them and 1 KiB of weights through the L1 per MT; a
+// CU's LDS (128 B/cycle) and L1 (64 B/cycle) keep the matrix cores busy only
+// from NT * NMAT = 2 and MT = 4 on.  So every shape has NT * NMAT = 2 but the
+// K-partitioned one, which is latency bound.  28-layer chunk, us per launch,
+// NT = 1 -> NT = 2: 2048 rows Q|K|V 31.7 -> 29.0, O 21.9 -> 15.0, down 24.0 ->
+// 18.0; 512 rows Q|K|V 12.4 -> 11.9.
 //
 // Tile order: workgroup i runs on XCD i % 8 (round-robin dispatch); the tiles
 // are numbered so that consecutive tiles share a column block (the same
@@ -77,7 +86,7 @@ __device__ __forceinline__ void xcd_tile(int id, int total, int tiles_m, int *n_
 // LDS address of A row r, 16-byte chunk c (chunks XOR-swizzled by row).
 __device__ __forceinline__ int a_off(int r, int c, int K) { return r * K + 16 * (c ^ (r & 7)); }
 
-template <int BM, int NWN, int KP, int NT, int NMAT, int D, int KB, int EPI, int GROUP, bool BSG>
+template <int BM, int NWN, int KP, int NT, int NMAT, int D, int KB, int EPI, int GROUP, bool BSG, int CB>
 __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) {
   using S = StreamShape<BM, NWN, KP, NT, NMAT, D, KB>;
   constexpr int MT = S::MT, K = S::K, NW = S::NW;
@@ -267,13 +276,13 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[mi][mt][nt][i] = 0.0f;
-  v4i c[2][NMAT][MT][NT];
+  v4i c[CB][NMAT][MT][NT];
 #pragma unroll
   for (int mi = 0; mi < NMAT; ++mi)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) c[0][mi][mt][nt] = c[1][mi][mt][nt] = zero4();
+      for (int nt = 0; nt < NT; ++nt) c[0][mi][mt][nt] = c[CB - 1][mi][mt][nt] = zero4();
 
   // every wave's A and scale copies are in LDS once slice 0 has arrived
   // (loads complete in order and the copies were issued first)
@@ -342,12 +351,13 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
         constexpr int j = decltype(J)::value;
         constexpr bool last = decltype(LAST)::value;
         constexpr int after = last ? (D - 1 < BODY - 1 - j ? D - 1 : BODY - 1 - j) : D - 1;
-        slice(std::integral_constant<int, j % D>{}, std::integral_constant<int, (j / SPG) & 1>{},
+        slice(std::integral_constant<int, j % D>{}, std::integral_constant<int, CB == 2 ? (j / SPG) & 1 : 0>{},
               std::integral_constant<int, after>{}, std::integral_constant<bool, !last || j + D < BODY>{},
               g0 * SPG + j);
         // at a group's first slice: the previous group, whose MFMAs are all
         // issued, is dequantised while these run
-        if constexpr (j % SPG == 0) {
+        if constexpr (CB == 1 && j % SPG == SPG - 1) dequant(std::integral_constant<int, 0>{}, g0 + j / SPG);
+        if constexpr (CB == 2 && j % SPG == 0) {
           const int g = g0 + j / SPG;
           if (g > 0) dequant(std::integral_constant<int, ((j / SPG) & 1) ^ 1>{}, g - 1);
         }
@@ -356,7 +366,7 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
 #pragma unroll 1
     for (int g0 = 0; g0 < NG - GPB; g0 += GPB) body(std::false_type{}, g0);
     body(std::true_type{}, NG - GPB);
-    dequant(std::integral_constant<int, (NG - 1) & 1>{}, NG - 1);
+    if constexpr (CB == 2) dequant(std::integral_constant<int, (NG - 1) & 1>{}, NG - 1);
   } else {
     // 3'. K partitions: the wave's GPP groups, each dequantised into a
     //     partial of its own (p = RN(RN(f32(I_g) * bs) * as)); then the
@@ -501,7 +511,7 @@ __global__ void __launch_bounds__(NWN * KP * 64) gemm_stream_kernel(TileArgs a) 
   }
 }
 
-template <int BM, int NWN, int KP, int NT, int NMAT, int D, int KB, int EPI, int GROUP, bool BSG>
+template <int BM, int NWN, int KP, int NT, int NMAT, int D, int KB, int EPI, int GROUP, bool BSG, int CB>
 hipError_t launch_one(const TileArgs &a, hipStream_t s) {
   using S = StreamShape<BM, NWN, KP, NT, NMAT, D, KB>;
   constexpr int NG = S::K / GROUP;
@@ -512,40 +522,59 @@ hipError_t launch_one(const TileArgs &a, hipStream_t s) {
   static bool attr_set = false;  // more than 64 KiB of dynamic LDS must be allowed once
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&gemm_stream_kernel<BM, NWN, KP, NT, NMAT, D, KB, EPI, GROUP, BSG>),
+        reinterpret_cast<const void *>(&gemm_stream_kernel<BM, NWN, KP, NT, NMAT, D, KB, EPI, GROUP, BSG, CB>),
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
   const int tiles = (a.N / S::BN) * ((a.M + BM - 1) / BM);
-  Q3_LAUNCH((gemm_stream_kernel<BM, NWN, KP, NT, NMAT, D, KB, EPI, GROUP, BSG>), dim3(tiles), dim3(S::NTHR), lds,
+  Q3_LAUNCH((gemm_stream_kernel<BM, NWN, KP, NT, NMAT, D, KB, EPI, GROUP, BSG, CB>), dim3(tiles), dim3(S::NTHR), lds,
             s, a);
   return hipGetLastError();
 }
 
-template <int BM, int NWN, int KP, int NT, int NMAT, int D, int EPI, bool BSG>
+template <int BM, int NWN, int KP, int NT, int NMAT, int D, int EPI, bool BSG, int CB = 2>
 hipError_t launch_k(const TileArgs &a, hipStream_t s) {
   const int kb = a.K / 1024;
   if (a.group == 256) {
-    if (kb == 1) return launch_one<BM, NWN, KP, NT, NMAT, D, 1, EPI, 256, BSG>(a, s);
-    if (kb == 2) return launch_one<BM, NWN, KP, NT, NMAT, D, 2, EPI, 256, BSG>(a, s);
-    if (kb == 3) return launch_one<BM, NWN, KP, NT, NMAT, D, 3, EPI, 256, BSG>(a, s);
+    if (kb == 1) return launch_one<BM, NWN, KP, NT, NMAT, D, 1, EPI, 256, BSG, CB>(a, s);
+    if (kb == 2) return launch_one<BM, NWN, KP, NT, NMAT, D, 2, EPI, 256, BSG, CB>(a, s);
+    if (kb == 3) return launch_one<BM, NWN, KP, NT, NMAT, D, 3, EPI, 256, BSG, CB>(a, s);
   } else if (a.group == 128) {
-    if (kb == 1) return launch_one<BM, NWN, KP, NT, NMAT, D, 1, EPI, 128, BSG>(a, s);
-    if (kb == 2) return launch_one<BM, NWN, KP, NT, NMAT, D, 2, EPI, 128, BSG>(a, s);
-    if (kb == 3) return launch_one<BM, NWN, KP, NT, NMAT, D, 3, EPI, 128, BSG>(a, s);
+    if (kb == 1) return launch_one<BM, NWN, KP, NT, NMAT, D, 1, EPI, 128, BSG, CB>(a, s);
+    if (kb == 2) return launch_one<BM, NWN, KP, NT, NMAT, D, 2, EPI, 128, BSG, CB>(a, s);
+    if (kb == 3) return launch_one<BM, NWN, KP, NT, NMAT, D, 3, EPI, 128, BSG, CB>(a, s);
   }
   return hipErrorInvalidValue;
 }
 
-// STORE / ADD: 16 waves per workgroup, as 8 column blocks x 2 K partitions
-// (128-column tiles) when those give at least one workgroup per CU, else
-// 4 column blocks x 4 K partitions (64-column tiles).
+// STORE / ADD: the smallest tiles whose grid is one workgroup per CU (256):
+// 64 columns as 4 column blocks x 4 K partitions, then 128 and 256 columns by
+// 8 waves over the whole of K (A tiles of K = 3072 leave room for one
+// workgroup per CU, so a grid just above 256 runs twice as long).  O (K =
+// 2048) / down (K = 3072) into 1024 columns, us a launch in a chunk: 512 rows
+// 8.8 / 9.4 in 64 columns, 10.4 / 11.2 in 128; 768 rows 12.9 / 14.9, 10.5 /
+// 12.1, 12.3 / 15.2 in 256; 1024 rows 11.3 / 13.2 in 128, 12.4 / 15.5 in 256;
+// 1536 rows 16.0 / 21.0, 13.8 / 16.5; 2048 rows 17.6 / 24.6, 15.0 / 18.0 (8
+// column blocks x 2 K partitions, 128 columns: 768 rows not taken, 1024 rows
+// 11.9 / 13.1, 2048 rows 21.9 / 24.0).
 template <int EPI, bool BSG>
 hipError_t launch_plain(const TileArgs &a, hipStream_t s) {
   const int tiles_m = (a.M + 31) / 32;
-  if (a.N % 128 == 0 && (a.N / 128) * tiles_m >= 256) return launch_k<32, 8, 2, 1, 1, 8, EPI, BSG>(a, s);
-  return launch_k<32, 4, 4, 1, 1, 4, EPI, BSG>(a, s);
+  if (a.N % 128 != 0 || (a.N / 64) * tiles_m <= 256) return launch_k<32, 4, 4, 1, 1, 4, EPI, BSG>(a, s);
+  if (a.N % 256 != 0 || (a.N / 128) * tiles_m <= 256) return launch_k<32, 8, 1, 1, 1, 8, EPI, BSG, 1>(a, s);
+  return launch_k<32, 8, 1, 2, 1, 8, EPI, BSG, 1>(a, s);
+}
+
+// Head epilogues: one 128-column head by 4 waves.  64-row tiles (K = 1024: two
+// workgroups per CU by LDS) from one full round of them on: Q|K|V (4096
+// columns), 32 / 64 rows a tile, us: 768 rows 14.1 / 14.8, 1024 rows 18.3 /
+// 16.1, 1536 rows 24.1 / 23.6, 2048 rows 29.0 / 29.0.
+template <int EPI>
+hipError_t launch_heads(const TileArgs &a, hipStream_t s) {
+  if (EPI == EPI_QKV && a.K == 1024 && a.group == 256 && (a.N / 128) * ((a.M + 63) / 64) >= 512)
+    return launch_one<64, 4, 1, 2, 1, 4, 1, EPI, 256, false, 1>(a, s);
+  return launch_k<32, 4, 1, 2, 1, 4, EPI, false>(a, s);
 }
 
 // One thread per 16-byte chunk of the packed matrix: chunk p = (fragment
@@ -598,15 +627,15 @@ hipError_t launch_gemm_stream(const TileArgs &a, int epi, hipStream_t s) {
   switch (epi) {
     case EPI_STORE: return a.bs_ld ? launch_plain<EPI_STORE, true>(a, s) : launch_plain<EPI_STORE, false>(a, s);
     case EPI_ADD: return a.bs_ld ? launch_plain<EPI_ADD, true>(a, s) : launch_plain<EPI_ADD, false>(a, s);
-    case EPI_HEADQ: return launch_k<32, 8, 1, 1, 1, 16, EPI_HEADQ, false>(a, s);
-    case EPI_NRQ: return launch_k<32, 8, 1, 1, 1, 16, EPI_NRQ, false>(a, s);
+    case EPI_HEADQ: return launch_heads<EPI_HEADQ>(a, s);
+    case EPI_NRQ: return launch_heads<EPI_NRQ>(a, s);
     case EPI_QKV:
       if (a.nseg < 1 || a.nseg > 3 || a.seg[0].n0 != 0 || a.seg[a.nseg - 1].n1 != a.N) return hipErrorInvalidValue;
       for (int i = 0; i < a.nseg; ++i)
         if (a.seg[i].n0 % 128 || a.seg[i].n1 % 128 || a.seg[i].n1 <= a.seg[i].n0 ||
             (i > 0 && a.seg[i].n0 != a.seg[i - 1].n1) || (reinterpret_cast<uintptr_t>(a.seg[i].b) & 15))
           return hipErrorInvalidValue;
-      return launch_k<32, 8, 1, 1, 1, 16, EPI_QKV, false>(a, s);
+      return launch_heads<EPI_QKV>(a, s);
     case EPI_SWIGLUQ: return launch_k<32, 16, 1, 1, 2, 4, EPI_SWIGLUQ, false>(a, s);
     default: return hipErrorInvalidValue;
   }
