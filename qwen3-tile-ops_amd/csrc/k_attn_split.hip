@@ -1,6 +1,7 @@
-// Decode attention with one sequence's keys over many workgroups, for long
-// contexts and small batches, bit-equal to the block walk of
-// kernels/attention_gqa.h:404-547 / ref_qwen3.py:210-266.
+// Attention with one sequence's keys over many workgroups, for decoding at long
+// contexts and in small batches and for short chunks at long contexts,
+// bit-equal to the block walk of kernels/attention_gqa.h:404-547 /
+// ref_qwen3.py:210-266.
 //
 // k_attn_decode.hip gives a sequence one workgroup per head (or per KV head),
 // which walks the key blocks chunk by chunk: a 4000-key context is six serial
@@ -269,6 +270,191 @@ __global__ void __launch_bounds__(kWaves * 64) split_pv_kernel(SplitArgs a) {
   }
 }
 
+// ---- several rows of one sequence (a short chunk) ---------------------------
+// The rows' int8 Q and K/V pages are there already, so both launches before
+// the chain work on (16-row tile, KV head, 4 blocks): PV = false the block
+// maxima of every row, PV = true the scores once more (four MFMAs a block cost
+// less than 2 KiB of scores through memory), then P, psum, P8 and P8.V.  Lane
+// layout of k_attn_prefill.hip: S^T = K.Q^T, lane (lc, lg) holds keys 16 kt +
+// 4 lg + i of row lc, whose P8 bytes are the B operand of V^T.P8^T.
+// What bounds it: latency at one tile (37 rows x 1040 keys: maxima 5.2, pv 12.2,
+// chain 7.0 us, the walk 24.6), the pv blocks (8 KiB a tile and head) through
+// memory from a few tiles on.  One query head per wave was faster for up to 8
+// rows (4000 keys 1574 against 1596 us a chunk) and slower from 37 on (2202
+// against 2112).
+constexpr int kTile = 16;
+
+template <bool PV>
+__global__ void __launch_bounds__(kWaves * 64) split_chunk_kernel(SplitArgs a) {
+  __shared__ uint64_t tab[32];
+  __shared__ __align__(16) int8_t vst[PV ? kWaves : 1][32 * HD];
+  __shared__ __align__(16) float scs[kWaves][64];
+  // ids with equal residues mod 8 (one XCD) take the KV heads and tiles of a run
+  const int ntiles = (a.rows + kTile - 1) / kTile;
+  const int id = static_cast<int>(blockIdx.x);
+  const int t = id >> 3;
+  const int kvh = t % a.kv_heads;
+  const int qi = t / a.kv_heads % ntiles * kTile;
+  const int b0 = (t / (a.kv_heads * ntiles) * 8 + (id & 7)) * kWaves;
+  const int nr = min(kTile, a.rows - qi);
+  const int kv_len = static_cast<int>(a.kv_len);
+  const int pos0 = kv_len - a.rows + qi;
+  const int nblk = (pos0 + nr + 31) / 32;
+  if (b0 >= nblk) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int lc = lane & 15, lg = lane >> 4;
+  const int blk = b0 + wave;
+  const int jb = min(blk, nblk - 1);
+  const int j = jb * 32;
+  const int row = qi + min(lc, nr - 1);  // (lanes past the tile's rows repeat the last)
+  const uint32_t page = a.table[static_cast<uint32_t>(j) / a.page_tokens];
+  const uint32_t slot0 = static_cast<uint32_t>(j) % a.page_tokens;
+  const int64_t koff = page * a.page_bytes + slot0 * a.row_bytes + kvh * HD;
+  if constexpr (PV) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 8 * e + (lane >> 3);
+      lds_copy16(a.v + koff + r * a.row_bytes + 16 * ((lane & 7) ^ vswz(r)), vst[wave] + 1024 * e);
+    }
+  }
+  v4i_d kop[2][2], qop[kGrp][2];
+  float qsv[kGrp];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      kop[kt][k] = *reinterpret_cast<const v4i_d *>(a.k + koff + (16 * kt + lc) * a.row_bytes + 16 * lg + 64 * k);
+#pragma unroll
+  for (int h = 0; h < kGrp; ++h) {
+    const int qh = kvh * kGrp + h;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      qop[h][k] = *reinterpret_cast<const v4i_d *>(a.q8 + row * a.ldq8 + qh * HD + 16 * lg + 64 * k);
+    qsv[h] = a.qs[row * a.ldqs + qh];
+  }
+  // lanes 0-31 the keys' ks, 32-63 their vs (0 past kv_len)
+  const int8_t *sb = reinterpret_cast<const int8_t *>(lane < 32 ? a.ks : a.vs) + page * a.scale_page_bytes +
+                     slot0 * a.scale_row_bytes;
+  const float scv = reinterpret_cast<const float *>(sb + (lane & 31) * a.scale_row_bytes)[kvh];
+  // row lc's maximum over the blocks before b0 (lane lg every fourth run), and
+  // the run's own blocks
+  float mrun[kGrp];
+  float4 grp[kGrp];
+  if constexpr (PV) {
+#pragma unroll
+    for (int h = 0; h < kGrp; ++h) {
+      const float *bm = a.ws_bmax + (static_cast<int64_t>(row) * a.heads + kvh * kGrp + h) * a.ldb;
+      grp[h] = *reinterpret_cast<const float4 *>(bm + b0);
+      float m = kFloor;
+      for (int i = 4 * lg; i < b0; i += 16) {
+        const float4 v = *reinterpret_cast<const float4 *>(bm + i);
+        m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+      }
+      mrun[h] = m;
+    }
+    if (threadIdx.x == 0) stage_exp2_table(tab);
+  }
+  float *sc = scs[wave];
+  sc[lane] = j + (lane & 31) < kv_len ? scv : 0.0f;
+  if constexpr (PV) {
+    wait_vmcnt<0>();  // the V copies have landed
+    __syncthreads();
+  }
+  if (blk >= nblk) return;
+  float ksr[2][4], vsr[2][4];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    const float4 k4 = *reinterpret_cast<const float4 *>(sc + 16 * kt + 4 * lg);
+    const float4 v4 = *reinterpret_cast<const float4 *>(sc + 32 + 16 * kt + 4 * lg);
+    ksr[kt][0] = k4.x, ksr[kt][1] = k4.y, ksr[kt][2] = k4.z, ksr[kt][3] = k4.w;
+    vsr[kt][0] = v4.x, vsr[kt][1] = v4.y, vsr[kt][2] = v4.z, vsr[kt][3] = v4.w;
+  }
+  const v4i_d z = {0, 0, 0, 0};
+  auto fold_max = [](float v) {  // over the four lanes of a row
+    LanePair p = lane_pair16(__float_as_uint(v));
+    v = fmaxf(__uint_as_float(p.a), __uint_as_float(p.b));
+    p = lane_pair32(__float_as_uint(v));
+    return fmaxf(__uint_as_float(p.a), __uint_as_float(p.b));
+  };
+#pragma unroll
+  for (int h = 0; h < kGrp; ++h) {
+    float s[2][4], bmax = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      v4i_d acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[kt][0], qop[h][0], z, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[kt][1], qop[h][1], acc, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = __fmul_rn(static_cast<float>(acc[i]), ksr[kt][i]);
+        x = __fmul_rn(x, qsv[h]);
+        x = __fmul_rn(x, a.qk_scale);
+        if (j + 16 * kt + 4 * lg + i > pos0 + lc) x = -INFINITY;
+        s[kt][i] = x;
+        bmax = fmaxf(bmax, x);
+      }
+    }
+    bmax = fold_max(bmax);
+    const int64_t wb = (static_cast<int64_t>(row) * a.heads + kvh * kGrp + h) * a.ldb + blk;
+    if constexpr (!PV) {
+      if (lg == 0 && lc < nr) a.ws_bmax[wb] = bmax;
+    } else {
+      float nmm = fmaxf(fold_max(mrun[h]), bmax);
+      if (wave > 0) nmm = fmaxf(nmm, grp[h].x);
+      if (wave > 1) nmm = fmaxf(nmm, grp[h].y);
+      if (wave > 2) nmm = fmaxf(nmm, grp[h].z);
+      float p[2][4], ts[2], pmx = 0.0f;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[kt][i] = exp_f32_le0_fast(__fsub_rn(s[kt][i], nmm), tab);
+        // the pairwise tree over the 32 keys: key bits 0-1 in registers, bits
+        // 2 and 3 over lg, bit 4 = kt
+        float u = __fadd_rn(__fadd_rn(p[kt][0], p[kt][1]), __fadd_rn(p[kt][2], p[kt][3]));
+        LanePair q = lane_pair16(__float_as_uint(u));
+        u = __fadd_rn(__uint_as_float(q.a), __uint_as_float(q.b));
+        q = lane_pair32(__float_as_uint(u));
+        ts[kt] = __fadd_rn(__uint_as_float(q.a), __uint_as_float(q.b));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          p[kt][i] = __fmul_rn(p[kt][i], vsr[kt][i]);
+          pmx = fmaxf(pmx, p[kt][i]);
+        }
+      }
+      const float pm = __fmul_rn(fold_max(pmx), inv127());
+      const double y = rcp64(pm);
+      uint32_t w8[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        w8[kt] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w8[kt] |= (static_cast<uint32_t>(quant_rcp(p[kt][i], y)) & 0xffu) << (8 * i);
+      }
+      if (lg == 0 && lc < nr) {
+        a.ws_psum[wb] = __fadd_rn(ts[0], ts[1]);
+        a.ws_nmm[wb] = nmm;
+      }
+      const long bp = static_cast<long>((static_cast<uint64_t>(w8[1]) << 32) | w8[0]);
+      const int jj = (lane & 15) >> 1;
+      const int key = 16 * (jj >> 2) + 4 * lg + (jj & 3);
+      const int8_t *vq = vst[wave] + key * HD + 8 * (lane & 1);
+      float *dst = a.ws_pv + wb * HD + 4 * lg;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        const v2i_d vt =
+            __builtin_amdgcn_ds_read_tr8_b64_v2i32(reinterpret_cast<lds_v2i_ptr_d>(to_lds(vq + ((dt ^ vswz(key)) << 4))));
+        long va;
+        __builtin_memcpy(&va, &vt, sizeof(va));
+        const v4i_d c = __builtin_amdgcn_mfma_i32_16x16x32_i8(va, bp, z, 0, 0, 0);
+        if (lc < nr)
+          *reinterpret_cast<float4 *>(dst + 16 * dt) =
+              make_float4(__fmul_rn(static_cast<float>(c[0]), pm), __fmul_rn(static_cast<float>(c[1]), pm),
+                          __fmul_rn(static_cast<float>(c[2]), pm), __fmul_rn(static_cast<float>(c[3]), pm));
+      }
+    }
+  }
+}
+
 constexpr int kChainWaves = 8;
 constexpr int kStage = 16;        // blocks per LDS stage (one instruction per wave)
 constexpr int kStages = 8;        // stages in flight
@@ -283,7 +469,7 @@ __global__ void __launch_bounds__(kChainWaves * 64) split_chain_kernel(SplitArgs
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = wave_id();
-  const uint32_t kv_len = a.row_pos ? static_cast<uint32_t>(a.row_pos[row]) + 1 : a.kv_len;
+  const uint32_t kv_len = a.row_pos ? static_cast<uint32_t>(a.row_pos[row]) + 1 : a.kv_len - (a.rows - 1 - row);
   const int nblk = static_cast<int>((kv_len + 31) / 32);
   const int64_t wb = (static_cast<int64_t>(row) * a.heads + qh) * a.ldb;
   if (tid == 0) stage_exp2_table(tab);
@@ -344,6 +530,10 @@ __global__ void __launch_bounds__(kChainWaves * 64) split_chain_kernel(SplitArgs
       lds_barrier();  // the stages are free again
     }
   }
+  // a chunk's rows walk to the end of their 32-row block's last row
+  // (ref_qwen3.py:281-288): fully masked blocks add +0 to res (-0 becomes +0)
+  if (!a.row_pos && static_cast<int>((kv_len + (min(row | 31, a.rows - 1) - row) + 31) / 32) > nblk)
+    res = __fadd_rn(res, 0.0f);
   // ---- epilogue: out = res * (1/den); per-head int8 quant (522-546) ----
   float out = 0.0f;
   if (wave < 2) {
@@ -391,6 +581,36 @@ hipError_t launch_attn_split(const SplitArgs &a, hipStream_t s) {
   if (grid >= (int64_t{1} << 31)) return hipErrorInvalidValue;
   Q3_LAUNCH(split_score_kernel, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), 0, s, a);
   Q3_LAUNCH(split_pv_kernel, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), 0, s, a);
+  Q3_LAUNCH(split_chain_kernel, dim3(static_cast<unsigned>(a.rows * a.heads)), dim3(kChainWaves * 64), 0, s, a);
+  return hipGetLastError();
+}
+
+bool attn_split_chunk_supported(const SplitArgs &a) {
+  if (!attn_split_supported(a) || a.row_pos || a.ldb % 4) return false;
+  if (a.kv_len < static_cast<uint32_t>(a.rows) || static_cast<int64_t>(a.max_blocks) * 32 < a.kv_len) return false;
+  auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  return al16(a.q8) && a.ldq8 % 16 == 0 && al16(a.ws_bmax);
+}
+
+// A chunk takes the split when the prefill kernel's walk (one workgroup per
+// 16-row tile and head, ~0.5 us per block) is long beside what every tile adds
+// to the split, its pv blocks through memory (~3 us a tile at 64 blocks).
+// 28-layer chunks, us (walk / split): 2 rows x 640 keys 1131 / 1148, 800 1235
+// / 1155, 2048 1804 / 1202, 4000 2790 / 1297; 16 x 800 1529 / 1491, 4000 3128
+// / 1716; 17 x 800 1558 / 1565, 1040 1685 / 1592; 37 x 1040 1722 / 1743, 1500
+// 1912 / 1849, 4000 3128 / 2112; 64 x 1040 1773 / 1818, 1500 1962 / 1939, 4000
+// 3172 / 2407; 96 x 2048 2402 / 2404, 128 x 2048 2393 / 2620.
+bool attn_split_chunk(int64_t rows, int64_t nblocks) {
+  return rows <= 64 && nblocks >= 17 + 8 * ((rows + kTile - 1) / kTile);
+}
+
+hipError_t launch_attn_split_chunk(const SplitArgs &a, hipStream_t s) {
+  if (!attn_split_chunk_supported(a)) return hipErrorInvalidValue;
+  const int64_t runs = (a.max_blocks + kWaves - 1) / kWaves, tiles = (a.rows + kTile - 1) / kTile;
+  const int64_t grid = (runs + 7) / 8 * 8 * a.kv_heads * tiles;
+  if (grid >= (int64_t{1} << 31)) return hipErrorInvalidValue;
+  Q3_LAUNCH(split_chunk_kernel<false>, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), 0, s, a);
+  Q3_LAUNCH(split_chunk_kernel<true>, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), 0, s, a);
   Q3_LAUNCH(split_chain_kernel, dim3(static_cast<unsigned>(a.rows * a.heads)), dim3(kChainWaves * 64), 0, s, a);
   return hipGetLastError();
 }

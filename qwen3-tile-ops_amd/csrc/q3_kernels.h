@@ -509,6 +509,12 @@ bool attn_split_supported(const SplitArgs &a);
 // whether a batch with these key blocks (longest row, all rows) takes it
 bool attn_split_batch(int64_t max_blocks, int64_t sum_blocks);
 hipError_t launch_attn_split(const SplitArgs &a, hipStream_t s);
+// The rows of one chunk (causal, the last at position kv_len - 1), whose Q rows
+// (q8, qs) and K/V pages hold the chunk already; ldb a multiple of 4.
+bool attn_split_chunk_supported(const SplitArgs &a);
+// whether a chunk of these rows and key blocks takes it
+bool attn_split_chunk(int64_t rows, int64_t nblocks);
+hipError_t launch_attn_split_chunk(const SplitArgs &a, hipStream_t s);
 
 // ---- greedy pick over a logits row (main_big.cpp:300-322) ---------------
 hipError_t launch_argmax_logits(const float *logits, int vocab,

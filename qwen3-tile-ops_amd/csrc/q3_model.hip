@@ -410,6 +410,21 @@ q3::SplitArgs split_args(const q3_model *m, const LayerPtrs &lp, int rows, uint3
   return a;
 }
 
+// The split attention of a chunk's last M rows (row tr0 of the stage rows on,
+// kv_len keys), when it applies and the sizes are its own.
+bool chunk_split_args(const q3_model *m, const LayerPtrs &lp, uint32_t kv_len, uint32_t tr0, int M,
+                      q3::SplitArgs *out) {
+  const int64_t nblocks = (kv_len + 31) / 32, ldb = (nblocks + 3) & ~int64_t{3};
+  if (!m->split_ws || M * ldb > m->split_blocks || !(m->split_always || q3::attn_split_chunk(M, nblocks))) return false;
+  q3::SplitArgs a = split_args(m, lp, M, kv_len, static_cast<int>(ldb));
+  a.q8 += tr0 * a.ldq8;
+  a.qs += tr0 * a.ldqs;
+  a.o8 += tr0 * a.ldo;
+  a.os += tr0 * a.ldos;
+  *out = a;
+  return q3::attn_split_chunk_supported(a);
+}
+
 // True when a chunk of `rows` runs on the decode-shaped kernels.
 bool small_path(const q3_layout &y, uint32_t rows) {
   const int H = static_cast<int>(y.hidden);
@@ -770,6 +785,8 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
     } else if (qkvfuse) {
       KTimer kt(m, Q3_KT_ATTN_DECODE);
       Q3_HIP(q3::launch_qkv_attn(gq, t, s));
+    } else if (q3::SplitArgs cs; rows > 1 && chunk_split_args(m, lp, pos + rows, tr0, M, &cs)) {
+      Q3_HIP(q3::launch_attn_split_chunk(cs, s));
     } else if (q3::attn_decode_supported(t)) {
       KTimer kt(m, Q3_KT_ATTN_DECODE);
       Q3_HIP(q3::launch_attn_decode(t, s));
@@ -1056,7 +1073,9 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
       t.os = os + static_cast<int64_t>(tr0) * y.heads;
       t.ldos = y.heads;
       t.os_col = 1;
-      if (q3::attn_decode_supported(t))
+      if (q3::SplitArgs cs; chunk_split_args(m, lp, pos + rows, tr0, M, &cs))
+        Q3_HIP(q3::launch_attn_split_chunk(cs, s));
+      else if (q3::attn_decode_supported(t))
         Q3_HIP(q3::launch_attn_decode(t, s));
       else
         Q3_HIP(q3::launch_attention(t, s));
@@ -1296,7 +1315,8 @@ extern "C" int q3_model_open(void *blob, const q3_layout *lay, void *stream, q3_
   m->split_always = split_env && std::atoi(split_env) == 1;
   if (lay->heads == 2 * lay->kv_heads && !(split_env && std::atoi(split_env) == 0)) {
     // without room for it the single-launch attention takes every length
-    m->split_blocks = std::min<int64_t>(kSplitMaxBlocks, static_cast<int64_t>(lay->seq) * m->n_pages);
+    // (a chunk's rows are a multiple of 4 blocks apart)
+    m->split_blocks = std::min<int64_t>(kSplitMaxBlocks, lay->seq * ((m->n_pages + int64_t{3}) & ~int64_t{3}));
     if (hipMalloc(&m->split_ws, sizeof(float) * static_cast<size_t>(lay->heads) * m->split_blocks * (128 + 32 + 3)) !=
         hipSuccess) {
       (void)hipGetLastError();

@@ -1,4 +1,4 @@
-"""The split decode attention (k_attn_split.hip: a sequence's key blocks over
+"""The split attention (k_attn_split.hip: a sequence's key blocks over
 many workgroups) at the edges of its blocks (32 keys), workgroups (4 blocks)
 and chain stages (16 blocks, 128 per pass), against the oracle in batches and
 against the single-launch attention for one row; and the one-row whole-row
@@ -144,3 +144,44 @@ def test_few_rows_whole_row_gemm(cuda, M, K, group, per_group):
     xt = dev(x)
     ops.gemm_nt_group_store(ta, tas, dev(b), dev(bs), None, group, add=xt)
     assert bits_equal(host(xt), (ref + x).astype(np.float32))
+
+
+def test_split_chunk_matches_tile_walk(cuda, monkeypatch):
+    """Short chunks at the edges of 16-row tiles, 32-row blocks, key blocks,
+    4-block workgroups and chain passes: logits of the last row and every
+    stage row equal the prefill kernel's, over a shuffled page table, with the
+    last layer on all rows and on the last one."""
+    shape = ModelShape(layers=2, vocab=1024, seq=64, max_seq=4352)
+    lay = Layout(shape)
+    blob = init_random_blob(lay, InitConfig(n_prompt=1, n_gen=0, mode=0))
+    rng = np.random.default_rng(11)
+    o, ms = lay.offsets, lay.max_seq
+    for li in range(shape.layers):
+        base = o["kKV_BASE"] + li * o["kKV_STRIDE"]
+        for off in (0, o["kKV_VOFF"]):
+            n = ms * lay.kv_width
+            blob[base + off:base + off + n] = rng.integers(-127, 128, n, dtype=np.int8).view(np.uint8)
+            so = base + off + o["kKV_SOFF"]
+            sc = rng.uniform(0.002, 0.03, ms * lay.kv_heads).astype(np.float32)
+            blob[so:so + 4 * sc.size] = sc.view(np.uint8)
+    table = rng.permutation(ms // 32).astype(np.uint16)
+    ids = rng.integers(0, 1024, ms).astype(np.int32)
+    chunks = [(0, 2), (30, 3), (127, 8), (4095, 2), (0, 9), (0, 64), (31, 16), (111, 17), (112, 16), (500, 33),
+              (1003, 37), (4032, 64), (4063, 33), (4351 - 32, 32)]
+    res = {}
+    for split in ("0", "1"):
+        monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+        m = Model(lay, blob)
+        m.set_page_table(table)
+        m.set_ids(ids)
+        for pos, rows in chunks:
+            for tail in (False, True):
+                m.forward_chunk(pos, rows, LM_LOGITS, tail)
+                res[split, pos, rows, tail] = ([m.stage("logits", 1)] +
+                                               [m.stage(nm, rows) for nm in ("x", "q8", "qs", "o8", "os")])
+        res[split, "kv"] = [m.kv_cache(li, ms)[nm] for li in range(2) for nm in ("kc", "ks", "vc", "vs")]
+        m.close()
+    for (split, *what), v in res.items():
+        if split == "1":
+            for a, b in zip(v, res[("0", *what)]):
+                assert bits_equal(a, b), (what, describe_diff(a, b))
