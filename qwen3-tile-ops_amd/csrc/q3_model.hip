@@ -811,14 +811,33 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
       KTimer kt(m, Q3_KT_GEMV_GATE_UP);
       Q3_HIP(q3::launch_gemv(gu, s));
     }
-    // down projection + residual; prologue = per-256 quant of SwiGLU
+    // down projection + residual; prologue (one row) = per-256 quant of SwiGLU
     {
       q3::GemvArgs g = gemv_args(M, I, 256);
-      g.pro = q3::PRO_QUANT;
-      g.x = sw + static_cast<int64_t>(tr0) * I;
-      g.ldx = I;
-      g.h8_out = s8 + static_cast<int64_t>(tr0) * I;
-      g.hs_out = ss + static_cast<int64_t>(tr0) * (I / 256);
+      if (M == 1) {
+        g.pro = q3::PRO_QUANT;
+        g.x = sw + static_cast<int64_t>(tr0) * I;
+        g.ldx = I;
+        g.h8_out = s8 + static_cast<int64_t>(tr0) * I;
+        g.hs_out = ss + static_cast<int64_t>(tr0) * (I / 256);
+      } else {  // several rows: as in q3_decode_batch
+        q3::RowArgs r{};
+        r.mode = 0;
+        r.rows = M;
+        r.cols = I;
+        r.x = sw + static_cast<int64_t>(tr0) * I;
+        r.ldx = I;
+        r.h8 = s8 + static_cast<int64_t>(tr0) * I;
+        r.ldh8 = I;
+        r.hs = ss + static_cast<int64_t>(tr0) * (I / 256);
+        r.ldhs = I / 256;
+        r.group = 256;
+        Q3_HIP(q3::launch_rows(r, s));
+        g.a = r.h8;
+        g.lda = I;
+        g.as = r.hs;
+        g.ldas = I / 256;
+      }
       g.nseg = 1;
       g.seg[0] = gemv_seg(0, H, q3::EPI_ADD, lp.wd, lp.wds, xt, H);
       if (ofuse) {  // x = (x + O) + down
@@ -1456,8 +1475,11 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
   // epilogues and the SwiGLU quantisation as launches of their own
   const bool gv = q3::gemv_rows_supported(M, H, 256, QW + 2 * KW) && q3::gemv_rows_supported(M, QW, HD, H) &&
                   q3::gemv_rows_supported(M, I, 256, H) && q3::gemv_rows_supported(M, H, 256, I);
-  // up to 8 rows: RMSNorm (layer 0: the embedding) and the quantisations run
-  // in the GEMVs' prologues
+  // up to 8 rows: RMSNorm (layer 0: the embedding) and its quantisation run in
+  // the GEMVs' prologues.  The SwiGLU rows' quantisation does not: down then
+  // takes one wave per weight row (28 layers, 300-600 keys, prologue / separate
+  // launch, us: 2 rows 992 / 964, 4 rows 1035 / 996, 5 rows 1167 / 1112, 8 rows
+  // 1249 / 1176)
   const bool pro = gv && small_path(y, n);
   if (!pro) Q3_TRY(rows(2, layer_ptrs(m, 0).n1));
   float *qf = at<float>(m, y.kQ), *kf = at<float>(m, y.kK), *vf = at<float>(m, y.kV);
@@ -1665,7 +1687,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       r.hs = ss;
       r.ldhs = I / 256;
       r.group = 256;
-      if (!pro) Q3_HIP(q3::launch_rows(r, s));
+      Q3_HIP(q3::launch_rows(r, s));
     } else {  // gate/up + SwiGLU + quant
       q3::GateUpArgs u;
       std::memset(&u, 0, sizeof(u));
@@ -1698,14 +1720,6 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       g.ldas = I / 256;
       g.nseg = 1;
       g.seg[0] = gemv_seg(0, H, q3::EPI_ADD, lp.wd, lp.wds, x, H);
-      if (pro) {  // quant256 of the SwiGLU rows
-        g.a = nullptr;
-        g.pro = q3::PRO_QUANT;
-        g.x = swf;
-        g.ldx = I;
-        g.h8_out = s8;
-        g.hs_out = ss;
-      }
       Q3_HIP(q3::launch_gemv(g, s));
     } else {
       q3::GemmArgs g = gemm_args(M, H, I, 256, s8, ss, lp.wd, lp.wds);
