@@ -285,12 +285,15 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
     if (g >= G || wave >= nb_of(1, g)) return;
     const int8_t *vb = pa.v + (static_cast<int64_t>(pg(page)) * pa.page_bytes + kvh * HD + slot_of(g) * rb);
     int8_t *dst = L.v[g & 1][wave];
-    // key 8 t + l3: vswz(key) = (l3 & 3) | (t & 2) << 1
+    // key 8 t + l3: vswz(key) = (l3 & 3) | (t & 2) << 1.  The chunk is swizzled
+    // before the row offset is added: a row may start at any multiple of 16,
+    // so bit 6 of the sum is not the chunk's.
     const uint32_t l3 = static_cast<uint32_t>(lane) >> 3;
-    const uint32_t off = l3 * rb + (((static_cast<uint32_t>(lane) & 7) ^ (l3 & 3)) << 4);
+    const uint32_t c16 = ((static_cast<uint32_t>(lane) & 7) ^ (l3 & 3)) << 4;
+    const uint32_t off[2] = {l3 * rb + c16, l3 * rb + (c16 ^ 64u)};
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int8_t *src = vb + (8u * t * rb) + (t < 2 ? off : off ^ 64u);
+      const int8_t *src = vb + (8u * t * rb) + off[t >> 1];
       __builtin_amdgcn_global_load_lds(const_cast<int8_t *>(src), to_lds(dst + t * 1024), 16, 0, 0);
     }
   };

@@ -46,3 +46,32 @@ def test_prefill_p8_half_integers(cuda, unit, nudge, rows, kv_len):
     ro8, ros = oracle.quant_rows_heads(attn, 128)
     assert bits_equal(host(o8), ro8), describe_diff(host(o8), ro8)
     assert bits_equal(host(os_), ros), describe_diff(host(os_), ros)
+
+
+@pytest.mark.parametrize("variant", ["", "pair", "walk"])
+@pytest.mark.parametrize("page_tokens", [32, 128])
+@pytest.mark.parametrize("rows,kv_len", [(2, 45), (33, 300), (301, 700)])
+@pytest.mark.parametrize("row_bytes,scale_cols", [(1040, 8), (1088, 9), (1152, 11)])
+def test_prefill_padded_rows(cuda, monkeypatch, variant, page_tokens, rows, kv_len, row_bytes, scale_cols):
+    """K/V rows at any multiple of 16 bytes, not of 128 (row_bytes wider than
+    the heads), and padded scale rows; the last head of the pool's last page
+    is read."""
+    monkeypatch.setenv("Q3_PREFILL_ATTN", variant)
+    rng = np.random.default_rng(row_bytes + rows + page_tokens)
+    heads, kvh, kw = 16, 8, 1024
+    n_pages = (kv_len + page_tokens - 1) // page_tokens
+    (k8, v8, ks, vs), (kp, vp, ksp, vsp, table) = make_pages(rng, kv_len, row_bytes, scale_cols, n_pages,
+                                                             page_tokens=page_tokens)
+    assert n_pages - 1 in table
+    q8 = rng.integers(-127, 128, (rows, heads * 128)).astype(np.int8)
+    qs = rng.uniform(1e-3, 5e-2, (rows, heads)).astype(F)
+    kv = ops.paged_kv(dev(kp), dev(vp), dev(ksp), dev(vsp), dev(table.view(np.int16)), page_tokens)
+    o8 = torch.zeros((rows, heads * 128), dtype=torch.int8, device=cuda)
+    os_ = torch.zeros((rows, heads), dtype=torch.float32, device=cuda)
+    ops.attention_heads_gqa_tokscale_paged(dev(q8), dev(qs), kv, kv_len, o8, os_, heads, kvh, 128, True, QK)
+    cols = lambda t, n: np.ascontiguousarray(t[:, :n])  # noqa: E731
+    attn = oracle.attention_heads_gqa_tokscale(q8, qs, cols(k8, kw), cols(ks, kvh), cols(v8, kw), cols(vs, kvh),
+                                               heads, kvh, 128, True, QK)
+    ro8, ros = oracle.quant_rows_heads(attn, 128)
+    assert bits_equal(host(o8), ro8), describe_diff(host(o8), ro8)
+    assert bits_equal(host(os_), ros), describe_diff(host(os_), ros)
