@@ -538,7 +538,10 @@ __global__ void __launch_bounds__(kChainWaves * 64) split_chain_kernel(SplitArgs
   float out = 0.0f;
   if (wave < 2) {
     out = __fmul_rn(res, __fdiv_rn(1.0f, den));
-    const float mx = max64(fabsf(out));
+    float mx = max64(fabsf(out));
+    // a chunk's row without a number (infinite or NaN scores) gets scale 0 as
+    // from k_attn_prefill.hip, a decoding row NaN as from k_attn_decode.hip
+    if (!a.row_pos && a.rows > 1) mx = fmaxf(mx, 0.0f);
     if (lane == 0) amax[wave] = mx;
   }
   wait_vmcnt<0>();

@@ -185,3 +185,45 @@ def test_split_chunk_matches_tile_walk(cuda, monkeypatch):
         if split == "1":
             for a, b in zip(v, res[("0", *what)]):
                 assert bits_equal(a, b), (what, describe_diff(a, b))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_split_special_scales(cuda, monkeypatch, value):
+    """Rows whose scores are infinite or NaN (K scales of the pool) come out
+    as from the kernels that take the same rows without the split: a chunk's
+    with scale 0, a decoding row's with scale NaN."""
+    lay = Layout(ModelShape(layers=1, vocab=1024, seq=64, max_seq=1024))
+    blob = init_random_blob(lay, InitConfig(n_prompt=1, n_gen=0, mode=0))
+    rng = np.random.default_rng(17)
+    o, ms = lay.offsets, lay.max_seq
+    for off in (0, o["kKV_VOFF"]):
+        at = o["kKV_BASE"] + off
+        n = ms * lay.kv_width
+        blob[at:at + n] = rng.integers(-127, 128, n, dtype=np.int8).view(np.uint8)
+        sc = rng.uniform(0.002, 0.03, ms * lay.kv_heads).astype(np.float32)
+        if off == 0:
+            sc.reshape(-1, lay.kv_heads)[40::300, ::2] = value
+        blob[at + o["kKV_SOFF"]:at + o["kKV_SOFF"] + 4 * sc.size] = sc.view(np.uint8)
+    ids = rng.integers(0, 1024, ms).astype(np.int32)
+    tables = np.tile(np.arange(ms // 32, dtype=np.uint16), (3, 1))
+    pos = np.array([20, 500, 1000], np.int32)
+    got = {}
+    for split in ("0", "1"):
+        monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+        m = Model(lay, blob)
+        m.set_ids(ids)
+        pool = m.blob.clone()
+        for at, rows in ((20, 2), (100, 16), (500, 37), (960, 64), (1000, 1)):
+            m.blob.copy_(pool)
+            m.forward_chunk(at, rows, LM_LOGITS, False)
+            got[split, at, rows] = m.stage("o8", rows), m.stage("os", rows)
+        m.blob.copy_(pool)
+        out = torch.zeros(3, dtype=torch.int32, device=cuda)
+        m.decode_batch(torch.from_numpy(ids[:3].copy()).to(cuda), pos, tables, out)
+        got[split, "batch"] = m.stage("o8", 3), m.stage("os", 3)
+        m.close()
+    for (split, *what), (o8, os_) in got.items():
+        if split == "1":
+            w8, ws = got[("0", *what)]
+            assert np.array_equal(o8, w8) and np.array_equal(os_, ws, equal_nan=True), what
+    assert np.isnan(got["1", 1000, 1][1]).any() and not np.isnan(got["1", 960, 64][1]).any()
