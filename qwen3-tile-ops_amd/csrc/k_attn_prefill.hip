@@ -480,10 +480,12 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
     const int nbA = g < G ? nb_of(0, g) : 0, nbB = g < G ? nb_of(1, g) : 0;
     const int j = g * CB + wave;
     wait_vmcnt<0>();  // this wave's copies and K rows of chunk g
-    float vsr[2][4];  // vs of keys 16 kt + 4 lg + i (0 past kv_len: P is 0 there)
+    float vsr[2][4];  // vs of keys 16 kt + 4 lg + i (0 past kv_len, where P is 0, and for NaN)
     if (wave < nbB) {
       float *sc = L.sc[wave];
-      sc[lane] = j * KB + (lane & 31) < kv_len ? scv : 0.0f;
+      // (a NaN vs as 0: its key's P8 is 0 either way, while the quantisation
+      // below would take the low byte of the NaN's payload)
+      sc[lane] = j * KB + (lane & 31) < kv_len && (lane < 32 || scv == scv) ? scv : 0.0f;
       float4 ks4[2];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {

@@ -48,6 +48,35 @@ def test_prefill_p8_half_integers(cuda, unit, nudge, rows, kv_len):
     assert bits_equal(host(os_), ros), describe_diff(host(os_), ros)
 
 
+@pytest.mark.parametrize("variant", ["", "pair"])
+@pytest.mark.parametrize("nan", [0x7FC00000, 0x7FC00055, 0xFFC00001])
+def test_prefill_nan_v_scale(cuda, monkeypatch, variant, nan):
+    """A key whose V scale is a NaN quantises to P8 = 0 whatever the NaN's
+    payload, in waves that otherwise take the approximate reciprocal."""
+    monkeypatch.setenv("Q3_PREFILL_ATTN", variant)
+    rng = np.random.default_rng(3)
+    rows, kv_len, heads, kvh = 33, 300, 16, 8
+    (k8, v8, ks, vs), (kp, vp, ksp, vsp, table) = make_pages(rng, kv_len, kvh * 128, kvh, 11)
+    q8 = rng.integers(-127, 128, (rows, heads * 128)).astype(np.int8)
+    qs = rng.uniform(1e-3, 5e-2, (rows, heads)).astype(F)
+    t = np.arange(5, kv_len, 41)
+    got = []
+    for special in (False, True):
+        # a NaN key's P * V is left out of the sum, as for a zero scale
+        vsp[table[t // 32], t % 32] = np.array([nan if special else 0], np.uint32).view(F)[0]
+        kv = ops.paged_kv(dev(kp), dev(vp), dev(ksp), dev(vsp), dev(table.view(np.int16)))
+        o8 = torch.zeros((rows, heads * 128), dtype=torch.int8, device=cuda)
+        os_ = torch.zeros((rows, heads), dtype=torch.float32, device=cuda)
+        ops.attention_heads_gqa_tokscale_paged(dev(q8), dev(qs), kv, kv_len, o8, os_, heads, kvh, 128, True, QK)
+        got.append((host(o8), host(os_)))
+    vs[t] = 0
+    attn = oracle.attention_heads_gqa_tokscale(q8, qs, k8, ks, v8, vs, heads, kvh, 128, True, QK)
+    ro8, ros = oracle.quant_rows_heads(attn, 128)
+    for o8, os_ in got:
+        assert bits_equal(o8, ro8), describe_diff(o8, ro8)
+        assert bits_equal(os_, ros), describe_diff(os_, ros)
+
+
 @pytest.mark.parametrize("variant", ["", "pair", "walk"])
 @pytest.mark.parametrize("page_tokens", [32, 128])
 @pytest.mark.parametrize("rows,kv_len", [(2, 45), (33, 300), (301, 700)])
