@@ -466,10 +466,10 @@ int q3_sched_run(q3_sched *s, q3_model *m, const q3_sched_item *items, uint32_t 
  * dispatch timestamps). */
 enum {
   Q3_KT_ATTN_DECODE = 0, /* decode attention (+ fused head epilogues)     */
-  Q3_KT_GEMV_QKV = 1,    /* Q|K|V projection, RMSNorm prologue            */
+  Q3_KT_GEMV_QKV = 1,    /* Q|K|V projection with its RMSNorm             */
   Q3_KT_GEMV_O = 2,      /* O projection + residual                       */
-  Q3_KT_GEMV_GATE_UP = 3,/* gate/up + SwiGLU, RMSNorm prologue            */
-  Q3_KT_GEMV_DOWN = 4,   /* down projection + residual, quant prologue    */
+  Q3_KT_GEMV_GATE_UP = 3,/* gate/up + SwiGLU with its RMSNorm             */
+  Q3_KT_GEMV_DOWN = 4,   /* down projection + residual with its quant     */
   Q3_KT_LM_HEAD = 5,     /* lm_head GEMV (argmax mode)                    */
   Q3_KT_COUNT = 6
 };
@@ -479,7 +479,12 @@ enum {
 int q3_model_set_kernel_timing(q3_model *m, uint32_t mask);
 
 /* Synchronises the stream and returns the summed milliseconds and the
- * number of timed launches of one class since timing was enabled. */
+ * number of timed launches of one class since timing was enabled.  Timed are
+ * q3_forward_chunk of up to 16 rows and q3_generate's decode steps (every
+ * class; the attention of single rows) and q3_decode_batch (the attention).
+ * What takes several kernels (the split attention, a norm or quant before a
+ * projection of several rows) counts as one launch, with the sum of their
+ * times. */
 int q3_model_kernel_time(q3_model *m, int kclass, double *total_ms, uint32_t *launches);
 
 #ifdef __cplusplus

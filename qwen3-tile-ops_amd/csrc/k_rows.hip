@@ -246,16 +246,15 @@ hipError_t launch_rows(const RowArgs &a, hipStream_t s) {
   if (quant_groups_ok(a)) {
     const int ngroups = a.cols / 256;
     const int64_t items = static_cast<int64_t>(a.rows) * ngroups;
-    hipLaunchKernelGGL(quant_groups_kernel, dim3(static_cast<unsigned>((items + 3) / 4)), dim3(256), 0, s, a,
-                       ngroups);
+    Q3_LAUNCH(quant_groups_kernel, dim3(static_cast<unsigned>((items + 3) / 4)), dim3(256), 0, s, a, ngroups);
     return hipGetLastError();
   }
   if (rows1024_ok(a)) {
-    hipLaunchKernelGGL(rows1024_kernel, dim3(a.rows), dim3(256), 0, s, a);
+    Q3_LAUNCH(rows1024_kernel, dim3(a.rows), dim3(256), 0, s, a);
     return hipGetLastError();
   }
   const dim3 grid((a.rows + 3) / 4);
-  hipLaunchKernelGGL(rows_kernel, grid, dim3(256), 0, s, a);
+  Q3_LAUNCH(rows_kernel, grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

@@ -11,20 +11,23 @@ namespace q3 {
 
 // ---- measurement hook ------------------------------------------------------
 // When set (by the model's kernel timing), the decode launchers time their
-// kernel with hipExtLaunchKernel start/stop events: the dispatch packet's own
-// timestamps, no extra queue packets.
+// kernels with hipExtLaunchKernel start/stop events: the dispatch packet's own
+// timestamps, no extra queue packets.  Each launch takes one pair of the list.
 struct LaunchEvents {
   hipEvent_t start, stop;
+  const LaunchEvents *next;
 };
 extern thread_local const LaunchEvents *g_launch_events;
 
 #define Q3_LAUNCH(kern, grid, block, shmem, stream, ...)                                      \
   do {                                                                                       \
-    if (::q3::g_launch_events)                                                               \
-      hipExtLaunchKernelGGL(kern, grid, block, shmem, stream, ::q3::g_launch_events->start,  \
-                            ::q3::g_launch_events->stop, 0, __VA_ARGS__);                    \
-    else                                                                                     \
+    if (const ::q3::LaunchEvents *q3_ev_ = ::q3::g_launch_events) {                          \
+      ::q3::g_launch_events = q3_ev_->next;                                                  \
+      hipExtLaunchKernelGGL(kern, grid, block, shmem, stream, q3_ev_->start, q3_ev_->stop, 0, \
+                            __VA_ARGS__);                                                    \
+    } else {                                                                                 \
       hipLaunchKernelGGL(kern, grid, block, shmem, stream, __VA_ARGS__);                     \
+    }                                                                                        \
   } while (0)
 
 // ---- row kernels: embedding gather, RMSNorm, per-group quantisation ----

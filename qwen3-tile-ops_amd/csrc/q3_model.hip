@@ -94,7 +94,7 @@ struct q3_model {
   std::vector<hipEvent_t> kt_ev[Q3_KT_COUNT];  // start, end pairs
   uint32_t kt_used[Q3_KT_COUNT] = {};          // pairs recorded
   double kt_ms[Q3_KT_COUNT] = {};              // folded totals
-  uint32_t kt_n[Q3_KT_COUNT] = {};
+  uint32_t kt_n[Q3_KT_COUNT] = {};             // calls timed (a call may be several launches)
   // decode: workgroups that prefetch the next kernels' weights during the
   // attention kernel (Q3_DECODE_PREFETCH_WGS, default 176; 0 disables)
   int pf_wgs;
@@ -129,6 +129,9 @@ constexpr uint32_t kPageTokens = 32;
 // workgroup, up to 8 rows together (28 layers, us, against the row kernels and
 // plain GEMVs: 2 rows 917 / 1050, 4 954 / 1053, 8 1134 / 1143, 9 1381 / 1173).
 constexpr int kMaxSmallRows = 8;
+// Rows of a chunk whose launches count for the kernel timing (Q3_KT_*): all of
+// forward_small's and those of forward_chunk_impl up to here.
+constexpr uint32_t kMaxTimedRows = 16;
 
 int hip_status(hipError_t e) { return e == hipSuccess ? Q3_OK : Q3_ERR_HIP; }
 
@@ -203,42 +206,47 @@ int kt_fold(q3_model *m, int c) {
     Q3_HIP(hipEventElapsedTime(&ms, m->kt_ev[c][2 * i], m->kt_ev[c][2 * i + 1]));
     m->kt_ms[c] += ms;
   }
-  m->kt_n[c] += m->kt_used[c];
   m->kt_used[c] = 0;
   return Q3_OK;
 }
 
-// Times the one launch issued during its lifetime, when class c is being
-// timed, through the launchers' hipExtLaunchKernel events.
+// Times the launches issued during its lifetime (the first n of them, 3 at
+// most) as one call of class c, when that class is being timed, through the
+// launchers' hipExtLaunchKernel events.
 class KTimer {
  public:
-  KTimer(q3_model *m, int c) : m_(m), c_(c) {
-    if (!(m->kt_mask & (1u << c))) return;
+  KTimer(q3_model *m, int c, uint32_t n = 1) : m_(m), c_(c), n_(std::min(n, kMaxLaunches)) {
+    if (n_ == 0 || !(m->kt_mask & (1u << c))) return;
     constexpr uint32_t kMaxPairs = 2048;
-    if (m->kt_used[c] == kMaxPairs && kt_fold(m, c) != Q3_OK) return;
+    if (m->kt_used[c] + n_ > kMaxPairs && kt_fold(m, c) != Q3_OK) return;
     std::vector<hipEvent_t> &ev = m->kt_ev[c];
-    while (ev.size() < 2 * (m->kt_used[c] + 1)) {
+    while (ev.size() < 2 * (m->kt_used[c] + n_)) {
       hipEvent_t e;
       if (hipEventCreate(&e) != hipSuccess) return;
       ev.push_back(e);
     }
-    pair_.start = ev[2 * m->kt_used[c]];
-    pair_.stop = ev[2 * m->kt_used[c] + 1];
-    q3::g_launch_events = &pair_;
+    for (uint32_t i = 0; i < n_; ++i)
+      pairs_[i] = {ev[2 * (m->kt_used[c] + i)], ev[2 * (m->kt_used[c] + i) + 1], i + 1 < n_ ? &pairs_[i + 1] : nullptr};
+    q3::g_launch_events = pairs_;
     active_ = true;
   }
   ~KTimer() {
     if (!active_) return;
+    const q3::LaunchEvents *left = q3::g_launch_events;
+    const uint32_t used = left ? static_cast<uint32_t>(left - pairs_) : n_;
     q3::g_launch_events = nullptr;
-    ++m_->kt_used[c_];
+    m_->kt_used[c_] += used;
+    m_->kt_n[c_] += used > 0;
   }
   KTimer(const KTimer &) = delete;
   KTimer &operator=(const KTimer &) = delete;
 
  private:
+  static constexpr uint32_t kMaxLaunches = 3;
   q3_model *m_;
   int c_;
-  q3::LaunchEvents pair_{};
+  uint32_t n_;
+  q3::LaunchEvents pairs_[kMaxLaunches] = {};
   bool active_ = false;
 };
 
@@ -778,6 +786,7 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
     }
     if (!do_tail) continue;
     if (split) {
+      KTimer kt(m, Q3_KT_ATTN_DECODE, 3);
       Q3_HIP(q3::launch_attn_split(split_args(m, lp, 1, pos + rows, static_cast<int>(nblocks)), s));
     } else if (merged) {
       KTimer kt(m, Q3_KT_ATTN_DECODE);
@@ -786,6 +795,7 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
       KTimer kt(m, Q3_KT_ATTN_DECODE);
       Q3_HIP(q3::launch_qkv_attn(gq, t, s));
     } else if (q3::SplitArgs cs; rows > 1 && chunk_split_args(m, lp, pos + rows, tr0, M, &cs)) {
+      KTimer kt(m, Q3_KT_ATTN_DECODE, M == 1 ? 3 : 0);  // (several rows: not a decode)
       Q3_HIP(q3::launch_attn_split_chunk(cs, s));
     } else if (q3::attn_decode_supported(t)) {
       KTimer kt(m, Q3_KT_ATTN_DECODE);
@@ -813,6 +823,7 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
     }
     // down projection + residual; prologue (one row) = per-256 quant of SwiGLU
     {
+      KTimer kt(m, Q3_KT_GEMV_DOWN, M == 1 ? 1 : 2);  // (nothing when offered to the next layer)
       q3::GemvArgs g = gemv_args(M, I, 256);
       if (M == 1) {
         g.pro = q3::PRO_QUANT;
@@ -849,7 +860,6 @@ int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int opti
         pend = g;
         have_pend = true;
       } else {
-        KTimer kt(m, Q3_KT_GEMV_DOWN);
         Q3_HIP(q3::launch_gemv(g, s));
       }
     }
@@ -1036,19 +1046,10 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
   float *ss = at<float>(m, y.kSS);
   const float qk_scale = static_cast<float>(1.0 / __builtin_sqrt(static_cast<double>(HD)));
 
-  // embedding + layer-0 RMSNorm (main_big.cpp:163-166), then its quant
-  {
-    const LayerPtrs l0 = layer_ptrs(m, 0);
-    const int rc = norm_quant_rows(m, 2, pos, 0, rows, l0.n1, x, h, h8, hs);
-    if (rc != Q3_OK) return rc;
-  }
-
+  // launches of the decode classes are timed in chunks of up to kMaxTimedRows
+  const uint32_t timed = rows <= kMaxTimedRows ? 1 : 0;
   for (uint32_t L = 0; L < y.layers; ++L) {
     const LayerPtrs lp = layer_ptrs(m, L);
-    if (L != 0) {
-      const int rc = norm_quant_rows(m, 1, pos, 0, rows, lp.n1, x, h, h8, hs);
-      if (rc != Q3_OK) return rc;
-    }
     // main_big.cpp:212-223: the last layer only needs the tail rows
     const bool is_last = (L + 1 == y.layers);
     const bool do_tail = !is_last || lm_out != Q3_LM_NONE;
@@ -1057,10 +1058,14 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
     const uint32_t tr = tail_last_row ? 1 : rows;
     const int M = static_cast<int>(tr);
 
-    // K (norm + RoPE + quant) and V (quant) straight into the page slots,
-    // Q (norm + RoPE + quant) for the tail rows
-    const int rc_qkv = qkv_projections(m, lp, pos, rows, do_tail, tr0, tr);
-    if (rc_qkv != Q3_OK) return rc_qkv;
+    // RMSNorm (layer 0: embedding + RMSNorm, main_big.cpp:163-166) + quant;
+    // K (norm + RoPE + quant) and V (quant) straight into the page slots, Q
+    // (norm + RoPE + quant) for the tail rows
+    {
+      KTimer kt(m, Q3_KT_GEMV_QKV, 2 * timed);
+      Q3_TRY(norm_quant_rows(m, L == 0 ? 2 : 1, pos, 0, rows, lp.n1, x, h, h8, hs));
+      Q3_TRY(qkv_projections(m, lp, pos, rows, do_tail, tr0, tr));
+    }
     if (!do_tail) continue;
 
     // paged GQA attention over kv_len = pos + rows keys
@@ -1092,6 +1097,7 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
       t.os = os + static_cast<int64_t>(tr0) * y.heads;
       t.ldos = y.heads;
       t.os_col = 1;
+      KTimer kt(m, Q3_KT_ATTN_DECODE, M == 1 ? 3 * timed : 0);
       if (q3::SplitArgs cs; chunk_split_args(m, lp, pos + rows, tr0, M, &cs))
         Q3_HIP(q3::launch_attn_split_chunk(cs, s));
       else if (q3::attn_decode_supported(t))
@@ -1113,6 +1119,7 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
       g.ldas = y.heads;
       g.nseg = 1;
       g.seg[0] = gemv_seg(0, H, q3::EPI_ADD, lp.wo, lp.wos, xt, H);
+      KTimer kt(m, Q3_KT_GEMV_O, timed);
       Q3_HIP(q3::launch_gemv(g, s));
     } else {
       q3::GemmArgs g = gemm_args(M, H, QW, HD, o8 + static_cast<int64_t>(tr0) * QW,
@@ -1127,13 +1134,12 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
         Q3_HIP(q3::launch_gemm(g, s));
       }
     }
-    // post-attention RMSNorm + quant
+    // post-attention RMSNorm + quant; gate/up + SwiGLU (+ quant, but on the
+    // GEMV tiles)
+    float *swf = at<float>(m, y.kSW) + static_cast<int64_t>(tr0) * I;
     {
-      const int rc = norm_quant_rows(m, 1, pos, tr0, tr, lp.n2, x, h, h8, hs);
-      if (rc != Q3_OK) return rc;
-    }
-    // gate/up + SwiGLU + quant
-    {
+      KTimer kt(m, Q3_KT_GEMV_GATE_UP, gv ? 2 * timed : 0);
+      Q3_TRY(norm_quant_rows(m, 1, pos, tr0, tr, lp.n2, x, h, h8, hs));
       q3::GateUpArgs u{};
       u.M = M;
       u.N = I;
@@ -1175,7 +1181,6 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
       t.ldss = I / 256;
       t.ss_col = 1;
       if (gv) {
-        float *swf = at<float>(m, y.kSW) + static_cast<int64_t>(tr0) * I;
         q3::GemvArgs g = gemv_args(M, H, 256);
         g.a = u.a;
         g.lda = H;
@@ -1186,18 +1191,6 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
         g.seg[0].b2 = lp.wu;
         g.seg[0].bs2 = lp.wus;
         Q3_HIP(q3::launch_gemv(g, s));
-        q3::RowArgs r{};
-        r.mode = 0;
-        r.rows = M;
-        r.cols = I;
-        r.x = swf;
-        r.ldx = I;
-        r.h8 = u.s8;
-        r.ldh8 = I;
-        r.hs = u.ss;
-        r.ldhs = I / 256;
-        r.group = 256;
-        Q3_HIP(q3::launch_rows(r, s));
       } else if (lp.pg && q3::gemm_stream_supported(t, q3::EPI_SWIGLUQ)) {
         Q3_HIP(q3::launch_gemm_stream(t, q3::EPI_SWIGLUQ, s));
       } else {
@@ -1206,10 +1199,23 @@ int forward_chunk_impl(q3_model *m, uint32_t pos, uint32_t rows, int lm_out,
     }
     // down projection + residual into x
     if (gv) {
+      KTimer kt(m, Q3_KT_GEMV_DOWN, 2 * timed);
+      q3::RowArgs r{};
+      r.mode = 0;
+      r.rows = M;
+      r.cols = I;
+      r.x = swf;
+      r.ldx = I;
+      r.h8 = s8 + static_cast<int64_t>(tr0) * I;
+      r.ldh8 = I;
+      r.hs = ss + static_cast<int64_t>(tr0) * (I / 256);
+      r.ldhs = I / 256;
+      r.group = 256;
+      Q3_HIP(q3::launch_rows(r, s));
       q3::GemvArgs g = gemv_args(M, I, 256);
-      g.a = s8 + static_cast<int64_t>(tr0) * I;
+      g.a = r.h8;
       g.lda = I;
-      g.as = ss + static_cast<int64_t>(tr0) * (I / 256);
+      g.as = r.hs;
       g.ldas = I / 256;
       g.nseg = 1;
       g.seg[0] = gemv_seg(0, H, q3::EPI_ADD, lp.wd, lp.wds, xt, H);
@@ -1530,6 +1536,7 @@ extern "C" int q3_decode_batch(q3_model *m, uint32_t n, const int32_t *ids, cons
       a.row_pos = m->bpos;
       a.table = m->btab;
       a.ld_table = ld_table;
+      KTimer kt(m, Q3_KT_ATTN_DECODE, 3);
       Q3_HIP(q3::launch_attn_split(a, s));
     } else if (gv) {
       q3::QkvHeadArgs e;

@@ -227,3 +227,38 @@ def test_split_special_scales(cuda, monkeypatch, value):
             w8, ws = got[("0", *what)]
             assert np.array_equal(o8, w8) and np.array_equal(os_, ws, equal_nan=True), what
     assert np.isnan(got["1", 1000, 1][1]).any() and not np.isnan(got["1", 960, 64][1]).any()
+
+
+@pytest.mark.parametrize("split", ["0", "1"])
+def test_split_kernel_timing(cuda, monkeypatch, split):
+    """Every route of the decode classes is timed, one launch per layer: the
+    split attention, projections of several rows with their norm or quant
+    kernel, chunks on both sides of the prologue GEMVs' row limit."""
+    monkeypatch.setenv("Q3_ATTN_SPLIT", split)
+    lay = Layout(ModelShape(layers=3, vocab=1024, seq=32, max_seq=2048))
+    m = Model(lay, init_random_blob(lay, InitConfig(n_prompt=1, n_gen=0, mode=0)))
+    m.set_ids(np.zeros(2048, np.int32))
+
+    def counts(call):
+        m.set_kernel_timing(True)
+        call()
+        kt = m.kernel_times()
+        m.set_kernel_timing(False)
+        assert all((ms > 0) == (n > 0) for ms, n in kt.values()), kt
+        return {k: n for k, (_, n) in kt.items()}
+
+    n = counts(lambda: m.forward_chunk(1600, 1, LM_LOGITS, True))
+    assert n["attn_decode"] == 3, n
+    if split == "1":
+        assert n["gemv_qkv"] == n["gemv_o"] == n["gemv_gate_up"] == n["gemv_down"] == 3, n
+    for rows in (4, 8, 9, 16):
+        for tail in (False, True):  # (the last layer's single row is a decode attention)
+            n = counts(lambda: m.forward_chunk(1000, rows, LM_LOGITS, tail))
+            assert n["attn_decode"] == int(tail), (rows, n)
+            assert n["gemv_qkv"] == n["gemv_o"] == n["gemv_gate_up"] == n["gemv_down"] == 3, (rows, n)
+    assert not any(counts(lambda: m.forward_chunk(1000, 17, LM_LOGITS, True)).values())
+    tables = np.stack([np.arange(64), np.arange(64)[::-1]]).astype(np.uint16)  # (no page of both in use)
+    out = torch.zeros(2, dtype=torch.int32, device=cuda)
+    n = counts(lambda: m.decode_batch(out, np.array([40, 1500], np.int32), tables, out))
+    assert n["attn_decode"] == 3, n
+    m.close()
