@@ -130,11 +130,16 @@ int gemm_common(const q3_view *a, const q3_view *a_scale, const q3_view *b,
 q3::GemvArgs to_gemv(const q3::GemmArgs &g);
 
 // The argmax over many columns only up to 8 rows: above, the tile kernel is
-// faster (151936 columns with the finish launch, 16 rows: 40.1 against 36.5
-// us; 8: 37.6), as long as its keys (one per 128 columns and row) fit the 4 MiB
-// workspace.
+// faster (with the finish launch, us, GEMV / tile: K = 1024 in groups of 256,
+// 151936 columns, 9 rows 33.4 / 30.5, 16 rows 34.8 / 30.3; K = 3072, 65536
+// columns, 9 rows 47.2 / 33.9), as long as its keys (one per 128 columns and
+// row) fit the 4 MiB workspace.  But K = 1024 in groups of 128 dequantises twice
+// as often on the tiles: 65536 columns, 9 rows 17.2 / 16.4, 100096 columns 23.7
+// / 24.7, 16 rows 24.9 / 24.7, 151936 columns 31.2 / 33.3 and 32.7 / 33.2.
 bool use_gemv(const q3::GemmArgs &g) {
-  if (g.epi == q3::EPI_ARGMAX && g.M > 8 && g.N >= 65536 && static_cast<int64_t>(g.N / 128) * g.M <= (1 << 19))
+  const bool tile_from_9 = g.K != 1024 || g.group != 128 || g.N < 98304;
+  if (g.epi == q3::EPI_ARGMAX && g.M > (tile_from_9 ? 8 : 16) && g.N >= 65536 &&
+      static_cast<int64_t>(g.N / 128) * g.M <= (1 << 19))
     return false;
   const bool shape = g.M <= 16 ? q3::gemv_supported(g.M, g.K, g.group)
                                : q3::gemv_rows_supported(g.M, g.K, g.group, g.N);

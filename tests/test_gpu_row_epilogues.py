@@ -88,3 +88,22 @@ def test_argmax_rows_and_ties(cuda, M, N, group):
     ref = oracle.gemm_nt_group(a, as_, b, bs, group)
     assert host(bidx)[:, 0].tolist() == [int(i) for i in np.argmax(ref, axis=1)]
     assert bits_equal(host(best)[:, 0], ref.max(axis=1))
+
+
+@pytest.mark.parametrize("N,group,M", [(65536, 128, 8), (65536, 128, 9), (98176, 128, 9), (98304, 128, 9),
+                                       (98304, 128, 16), (98304, 128, 17), (98304, 256, 9)])
+def test_argmax_wide_routes(cuda, N, group, M):
+    """Both sides of the rules that share a wide argmax out between the GEMV
+    and the tile kernel (rows, columns, group), with equal maxima."""
+    rng = np.random.default_rng(M + N)
+    a, as_, b, bs = rand_gemm(rng, M, 1024, N, group)
+    for src in range(0, N, 997):
+        for dst in (src + 1, src + 65, src + 50000):
+            if dst < N:
+                b[dst], bs[dst] = b[src], bs[src]
+    best = torch.full((M, 1), -3.0e38, dtype=torch.float32, device=cuda)
+    bidx = torch.zeros((M, 1), dtype=torch.int32, device=cuda)
+    ops.gemm_nt_group_argmax(dev(a), dev(as_), dev(b), dev(bs), best, bidx, group)
+    ref = oracle.gemm_nt_group(a, as_, b, bs, group)
+    assert host(bidx)[:, 0].tolist() == [int(i) for i in np.argmax(ref, axis=1)]
+    assert bits_equal(host(best)[:, 0], ref.max(axis=1))
