@@ -22,11 +22,12 @@
 //   PRO_EMBED  embedding gather + dequant (embedding.h:99-168), then as NORM
 //   PRO_QUANT  per-256 quant only (quant.h:89-138)
 // with the reference's exact rounding points; workgroup 0 also stores the
-// stage buffers (x, h, h8, hs) the reference writes.
+// stage buffers (x, h, h8, hs) the reference writes.  Up to 8 rows, PRO_QUANT
+// one.
 //
 // Epilogues: STORE, ADD (residual, group_gemm.h:194-214), SWIGLU (gate and up
 // rows of the same columns, swiglu_quant.h:195-231, stored as f32 for the
-// next prologue) and ARGMAX (lm_argmax.h:55-67: one (max, first index) key
+// next prologue or quant launch) and ARGMAX (lm_argmax.h:55-67: one (max, first index) key
 // per workgroup and row into a slot array, reduced by argmax_finish).
 #include <algorithm>
 
@@ -53,8 +54,8 @@ constexpr int kPartPro = 1, kPartEpi = 2;
 // the other scales before the weight stream (PRO_NONE, one matrix).
 // MT row tiles of 16 (MT > 1: plain A operand, rows past M computed on row
 // M - 1's data and not stored), their A fragments loaded AB tiles at a time.
-// RB: rows whose prologue operands are loaded and computed together
-// (pro_compute_rows; 1: one row, pro_compute_row).
+// RB > 1: up to RB rows, whose prologue operands are loaded and computed
+// together (pro_compute_rows; 1: one row, pro_compute_row).
 template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT,
           int RB = 1>
 __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
@@ -263,6 +264,8 @@ __global__ void __launch_bounds__(256) gemv_kernel(GemvArgs a) {
   if constexpr (PRO != PRO_NONE) {
     if constexpr (RB > 1) {
       pro_compute_rows<PRO, QW, RB>(a, 0, M, rb, a_lds, as_lds, blk, blockIdx.x == 0);
+      // (not entered, as M <= RB: without the loop the compiler schedules the
+      // rows worse, a batched step of 8 rows 1069 against 1053 us)
       for (int m0 = RB; m0 < M; m0 += RB) {
         pro_load_rows<PRO, QW, RB>(a, ps, m0, M, rb);
         pro_compute_rows<PRO, QW, RB>(a, m0, M, rb, a_lds, as_lds, blk, blockIdx.x == 0);
@@ -927,7 +930,7 @@ __global__ void __launch_bounds__(256) qkv_heads_kernel(QkvHeadArgs a) {
 template <int GPW, int KSTEPS, int NT, int NMAT, int PRO, int PART, bool BSG = false, int MT = 1, int AB = MT,
           int RB = 1>
 hipError_t launch_t(const GemvArgs &a, int ncols, hipStream_t s, int ry = 1) {
-  if (PRO != PRO_NONE && RB == 1 && a.M != 1) return hipErrorInvalidValue;
+  if (PRO != PRO_NONE && a.M > RB) return hipErrorInvalidValue;
   constexpr int NB = 16 * NT;
   // the prologue gives each wave GPW * KSTEPS / 4 groups of 256 columns
   if (PRO != PRO_NONE && a.K != 256 * GPW * KSTEPS) return hipErrorInvalidValue;
@@ -1000,8 +1003,11 @@ template <int NMAT, int PRO>
 hipError_t dispatch_pro(const GemvArgs &a, int ncols, hipStream_t s) {
   if (a.group != 256) return hipErrorInvalidValue;
   if (a.M == 1) return dispatch_pro_rows<NMAT, PRO, 1>(a, ncols, s);
-  if (a.M > 4 && a.M <= 8) return dispatch_pro_rows<NMAT, PRO, 8>(a, ncols, s);
-  return dispatch_pro_rows<NMAT, PRO, 4>(a, ncols, s);  // (16 rows of K = 3072 and eight rows' sums exceed 64 KiB)
+  if constexpr (PRO != PRO_QUANT) {  // (several rows are quantised by a launch of their own)
+    if (a.M <= 4) return dispatch_pro_rows<NMAT, PRO, 4>(a, ncols, s);
+    if (a.M <= 8) return dispatch_pro_rows<NMAT, PRO, 8>(a, ncols, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int NT, int NMAT>

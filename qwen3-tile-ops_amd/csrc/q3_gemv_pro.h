@@ -256,15 +256,15 @@ __device__ void pro_compute_row(const GemvArgs &a, int m, const ProRow<QW, NP> &
   lds_barrier();  // blk is reused by the next row; A is complete
 }
 
-// ---- RB rows at once (2 .. 16 rows of a chunk or batch) ------------------
-// pro_load_row / pro_compute_row for rows m0 .. m0 + RB - 1 (those past M
-// repeat row M - 1 and are not stored): all operands are requested together,
-// one barrier pair serves all rows, lane r computes row r's norm factor, and
-// lane r QW + q the f64 reciprocal of its (row, group) scale.
+// ---- RB rows at once (2 .. 8 rows of a chunk or batch) -------------------
+// pro_load_row / pro_compute_row of PRO_NORM and PRO_EMBED for rows m0 .. m0 +
+// RB - 1 (those past M repeat row M - 1 and are not stored): all operands are
+// requested together, one barrier pair serves all rows, lane r computes row r's
+// norm factor, and lane r QW + q the f64 reciprocal of its (row, group) scale.
 template <int PRO, int QW, int RB>
 struct ProRows {
   float4 x[RB][PRO == PRO_EMBED ? 1 : QW];
-  float4 w[PRO == PRO_QUANT ? 1 : QW];
+  float4 w[QW];
   uint32_t e[PRO == PRO_EMBED ? RB : 1][QW];
   float esc[PRO == PRO_EMBED ? RB : 1];
 };
@@ -293,10 +293,8 @@ __device__ __forceinline__ void pro_load_rows(const GemvArgs &a, const ProSrc &p
         r.x[i][q] = *reinterpret_cast<const float4 *>(ps.x + static_cast<int64_t>(m) * ps.ldx + c);
     }
   }
-  if constexpr (PRO != PRO_QUANT) {
 #pragma unroll
-    for (int q = 0; q < QW; ++q) r.w[q] = *reinterpret_cast<const float4 *>(ps.w + (wave + 4 * q) * 256 + 4 * lane);
-  }
+  for (int q = 0; q < QW; ++q) r.w[q] = *reinterpret_cast<const float4 *>(ps.w + (wave + 4 * q) * 256 + 4 * lane);
 }
 
 // floats of LDS that pro_compute_rows needs for its block sums
@@ -308,6 +306,7 @@ constexpr int pro_rows_blk() {
 template <int PRO, int QW, int RB>
 __device__ void pro_compute_rows(const GemvArgs &a, int m0, int M, const ProRows<PRO, QW, RB> &r, int8_t *a_lds,
                                  float *as_lds, float *blk, bool stage_writer) {
+  static_assert(PRO == PRO_NORM || PRO == PRO_EMBED, "RMSNorm rows");
   static_assert(RB * QW <= 64, "one lane per (row, group)");
   constexpr int NGR = 4 * QW, PITCH = 32 * QW + 4;
   const int lane = threadIdx.x & 63;
@@ -332,40 +331,38 @@ __device__ void pro_compute_rows(const GemvArgs &a, int m0, int M, const ProRows
         v[i][q][3] = r.x[i][q].w;
       }
     }
-  if constexpr (PRO != PRO_QUANT) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
+  for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int q = 0; q < QW; ++q) {
-        const float *x = v[i][q];
-        float s = __fadd_rn(__fadd_rn(__fmul_rn(x[0], x[0]), __fmul_rn(x[1], x[1])),
-                            __fadd_rn(__fmul_rn(x[2], x[2]), __fmul_rn(x[3], x[3])));
-        s = __fadd_rn(s, lane_xor<1>(s));
-        s = __fadd_rn(s, lane_xor<2>(s));
-        s = __fadd_rn(s, lane_xor<4>(s));
-        if ((lane & 7) == 0) blk[i * PITCH + (wave + 4 * q) * 8 + (lane >> 3)] = s;
-      }
-    lds_barrier();
-    float ss = 0.0f;
-    const float *br = blk + (lane % RB) * PITCH;
-#pragma unroll
-    for (int b = 0; b < 32 * QW; b += 4) {
-      const float4 b4 = *reinterpret_cast<const float4 *>(br + b);
-      ss = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(ss, b4.x), b4.y), b4.z), b4.w);
+    for (int q = 0; q < QW; ++q) {
+      const float *x = v[i][q];
+      float s = __fadd_rn(__fadd_rn(__fmul_rn(x[0], x[0]), __fmul_rn(x[1], x[1])),
+                          __fadd_rn(__fmul_rn(x[2], x[2]), __fmul_rn(x[3], x[3])));
+      s = __fadd_rn(s, lane_xor<1>(s));
+      s = __fadd_rn(s, lane_xor<2>(s));
+      s = __fadd_rn(s, lane_xor<4>(s));
+      if ((lane & 7) == 0) blk[i * PITCH + (wave + 4 * q) * 8 + (lane >> 3)] = s;
     }
-    const float rinv = rms_factor(ss, a.inv_pre);
+  lds_barrier();
+  float ss = 0.0f;
+  const float *br = blk + (lane % RB) * PITCH;
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      const float ri = lane_read(rinv, i);
+  for (int b = 0; b < 32 * QW; b += 4) {
+    const float4 b4 = *reinterpret_cast<const float4 *>(br + b);
+    ss = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(ss, b4.x), b4.y), b4.z), b4.w);
+  }
+  const float rinv = rms_factor(ss, a.inv_pre);
 #pragma unroll
-      for (int q = 0; q < QW; ++q) {
-        const float w4[4] = {r.w[q].x, r.w[q].y, r.w[q].z, r.w[q].w};
+  for (int i = 0; i < RB; ++i) {
+    const float ri = lane_read(rinv, i);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[i][q][t] = __fmul_rn(__fmul_rn(v[i][q][t], ri), w4[t]);
-        if (stage_writer && a.h_out && m0 + i < M)
-          *reinterpret_cast<float4 *>(a.h_out + static_cast<int64_t>(m0 + i) * K + (wave + 4 * q) * 256 + 4 * lane) =
-              make_float4(v[i][q][0], v[i][q][1], v[i][q][2], v[i][q][3]);
-      }
+    for (int q = 0; q < QW; ++q) {
+      const float w4[4] = {r.w[q].x, r.w[q].y, r.w[q].z, r.w[q].w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[i][q][t] = __fmul_rn(__fmul_rn(v[i][q][t], ri), w4[t]);
+      if (stage_writer && a.h_out && m0 + i < M)
+        *reinterpret_cast<float4 *>(a.h_out + static_cast<int64_t>(m0 + i) * K + (wave + 4 * q) * 256 + 4 * lane) =
+            make_float4(v[i][q][0], v[i][q][1], v[i][q][2], v[i][q][3]);
     }
   }
   float mine = 0.0f;  // lane i QW + q: absmax of row i, group wave + 4 q

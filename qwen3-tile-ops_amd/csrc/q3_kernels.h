@@ -358,8 +358,9 @@ hipError_t launch_nrq_rows(const NrqArgs &a, hipStream_t s);
 
 // ---- decode-shaped group GEMM (M <= 64) ---------------------------------
 // One launch can cover up to three column ranges with their own weights and
-// epilogue (fused Q/K/V).  No grid-wide synchronisation.  Prologues, O
-// partials and the lm_head's column streaming take at most 16 rows.
+// epilogue (fused Q/K/V).  No grid-wide synchronisation.  The RMSNorm
+// prologues take at most 8 rows, PRO_QUANT and the O partials one, the
+// lm_head's column streaming 16.
 enum Pro : int {
   PRO_NONE = 0,   // A operand int8 + scales from global memory
   PRO_NORM = 1,   // A = quant256(rmsnorm(x, w_pre))
