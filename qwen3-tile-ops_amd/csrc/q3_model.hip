@@ -127,7 +127,9 @@ constexpr uint32_t kPageTokens = 32;
 // Rows of a chunk (forward_small) or of a batch on the GEMVs with prologues,
 // which save the norm and quant launches but rebuild the int8 rows in every
 // workgroup, up to 8 rows together (28 layers, us, against the row kernels and
-// plain GEMVs: 2 rows 917 / 1050, 4 954 / 1053, 8 1134 / 1143, 9 1381 / 1173).
+// plain GEMVs: chunks of 2 rows 904 / 1047, 4 912 / 1063, 8 1047 / 1141, 9 1187 /
+// 1177, 16 1342 / 1198; batches at 300-600 keys of 2 rows 964 / 1118, 8 1173 /
+// 1238, 9 1328 / 1297; 9 and more rows were taken four at a time).
 constexpr int kMaxSmallRows = 8;
 // Rows of a chunk whose launches count for the kernel timing (Q3_KT_*): all of
 // forward_small's and those of forward_chunk_impl up to here.
@@ -484,10 +486,10 @@ int lm_head(q3_model *m, uint32_t rows, int lm_out, int32_t *id_dst) {
   return Q3_OK;
 }
 
-// main_big.cpp:145-296 for chunks of at most 16 rows: every GEMM is a
+// main_big.cpp:145-296 for chunks of at most kMaxSmallRows rows: every GEMM is a
 // whole-chip GEMV whose prologue builds its int8 operand from the f32 rows
-// (embedding / RMSNorm / quant), and whose epilogue is a plain store, the
-// residual add, SwiGLU or the argmax.
+// (embedding / RMSNorm, for one row also the quant of SwiGLU), and whose
+// epilogue is a plain store, the residual add, SwiGLU or the argmax.
 int forward_small(q3_model *m, uint32_t pos, uint32_t rows, int lm_out, int optimize_tail,
                   int32_t *id_dst) {
   const q3_layout &y = m->lay;
