@@ -76,6 +76,7 @@ def build(jobs: int = 0, verbose: bool = False) -> Path:
           *map(str, objs), "-pthread"])
     os.replace(tmp, OUT)
     build_c_driver()
+    build_device_math()
     if verbose:
         print(f"built {OUT}")
     return OUT
@@ -97,6 +98,19 @@ def build_c_driver() -> Path | None:
           f"-L{OUT.parent}", "-lq3ops", f"-L{ROCM / 'lib'}", "-lamdhip64",
           f"-Wl,-rpath,$ORIGIN/{rel}:{ROCM / 'lib'}", "-o", str(C_DRIVER)])
     return C_DRIVER
+
+
+DEVICE_MATH_SRC = REPO / "tests" / "device_math" / "device_math.hip"
+
+
+def build_device_math() -> Path | None:
+    """The device header's scalar functions as a library that the GPU tests
+    run over all of their ranges."""
+    if not DEVICE_MATH_SRC.exists():
+        return None
+    out = DEVICE_MATH_SRC.parent / "libdevice_math.so"
+    _run([str(ROCM / "bin" / "hipcc"), *HIP_FLAGS, "-shared", str(DEVICE_MATH_SRC), "-o", str(out)])
+    return out
 
 
 def main() -> int:

@@ -231,8 +231,8 @@ __device__ __forceinline__ float exp_f32_le0_tab(float x, const uint64_t *tab) {
 // (-151 <= x2 <= 200 or NaN).  The reduction in f32: x2 + 1.5 * 2^18 rounds x2 to
 // a multiple of 1/32 as glibc's f64 x2 + 1.5 * 2^47 does (|x2| < 2^17), and
 // r = x2 - k/32 is exact in f32.  Equal to glibc's exp2f on every float of the
-// range (checked exhaustively): 2^-150 and below round to +0, 2^128 and above
-// to +inf.
+// range (oracle/exp2_check.c, tests/test_gpu_device_math.py): 2^-150 and below
+// round to +0, 2^128 and above to +inf.
 __device__ __forceinline__ float exp2f_fast(float x2, const uint64_t *tab) {
   const float shift = 0x1.8p+18f;
   const float kf = __fadd_rn(x2, shift);
@@ -255,7 +255,9 @@ __device__ __forceinline__ float exp_f32_le0_fast(float x, const uint64_t *tab) 
 }
 
 // RN(1 / d) for 1 <= d < 2^126: v_rcp_f32 and one Newton step, equal to the
-// IEEE quotient for all 2^23 significands (checked exhaustively on gfx950).
+// IEEE quotient for all 2^23 significands (tests/test_gpu_device_math.py).  It
+// holds through what gfx950's v_rcp_f32 returns: from other reciprocals within
+// an ulp a few significands would come out an ulp off.
 __device__ __forceinline__ float rcp_ge1(float d) {
   const float r = __builtin_amdgcn_rcpf(d);
   return __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
