@@ -262,3 +262,25 @@ def test_split_kernel_timing(cuda, monkeypatch, split):
     n = counts(lambda: m.decode_batch(out, np.array([40, 1500], np.int32), tables, out))
     assert n["attn_decode"] == 3, n
     m.close()
+
+
+def test_split_chunk_matches_oracle(cuda, monkeypatch):
+    """A prompt in short chunks, all of them on the split attention, against
+    the oracle: the last layer's attention output and residual rows of every
+    chunk, and the logits."""
+    monkeypatch.setenv("Q3_ATTN_SPLIT", "1")
+    shape = ModelShape(layers=2, vocab=1024, seq=64, max_seq=640)
+    lay = Layout(shape)
+    blob = init_random_blob(lay, InitConfig(n_prompt=600, n_gen=0, mode=0))
+    om = oracle.OracleModel(blob, lay.offsets, dict(shape.__dict__))
+    ids = lay.global_views(blob)["ids"][:600].copy()
+    m = Model(lay, blob)
+    pos = 0
+    for rows in (64, 33, 2, 17, 9, 64, 16, 8, 3, 40, 64, 48, 5, 31, 64, 61, 24, 11):
+        logits, rec = om.forward_chunk(ids[pos:pos + rows], pos, rows, True, record=True)
+        m.forward_chunk(pos, rows, LM_LOGITS, False)
+        assert bits_equal(m.stage("logits", 1)[0], logits), (pos, rows)
+        for st in ("x", "o8", "os"):
+            assert bits_equal(m.stage(st, rows), rec[st]), (pos, rows, st)
+        pos += rows
+    m.close()

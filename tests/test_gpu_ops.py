@@ -609,9 +609,8 @@ def test_gemm_row_tiles(cuda, case, M, K, N, group):
 @pytest.mark.parametrize("M", [2, 5, 16, 20, 33, 64, 100])
 def test_lm_argmax_wide_multirow(cuda, M):
     """lm_head width with several rows: one running key per row and
-    workgroup across the column tiles each workgroup walks (M <= 16), one key
-    per row and 128-column tile of the LDS-staged tile kernel (M <= 64), and
-    the per-32-row kernel beyond."""
+    workgroup across the column tiles each workgroup walks (M <= 8), one key
+    per row and 128-column tile of the LDS-staged tile kernel beyond."""
     note(f"lm argmax M={M} N=151936")
     rng = np.random.default_rng(40 + M)
     a, as_, b, bs = rand_gemm(rng, M, 1024, 151936, 256)

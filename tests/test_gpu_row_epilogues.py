@@ -72,10 +72,13 @@ def test_gate_up_rows_and_range(cuda, M, off, scale):
 
 @pytest.mark.parametrize("M", [2, 9, 16, 17, 32, 33, 64, 65, 256])
 @pytest.mark.parametrize("N,group", [(128, 256), (1152, 256), (2176, 128)])
-def test_argmax_rows_and_ties(cuda, M, N, group):
-    """One key per row and 128-column tile for every row count of the tile
-    kernel (row tiles of 32 and 64), tile counts that are not a multiple of 8,
-    and equal maxima in one tile and across tiles: the first column wins."""
+@pytest.mark.parametrize("padded", [False, True])
+def test_argmax_rows_and_ties(cuda, M, N, group, padded):
+    """One key per row and 128-column tile of the tile kernel (row tiles of 32
+    and 64; padded weight rows, which the GEMV does not take, or more than 64
+    rows), tile counts that are not a multiple of 8, and equal maxima in one
+    tile and across tiles: the first column wins.  Up to 64 rows of dense
+    weights the GEMV's keys."""
     rng = np.random.default_rng(M + N)
     a, as_, b, bs = rand_gemm(rng, M, 1024, N, group)
     for src in range(0, N, 37):  # copies of rows, later in the tile and in other tiles
@@ -84,7 +87,9 @@ def test_argmax_rows_and_ties(cuda, M, N, group):
                 b[dst], bs[dst] = b[src], bs[src]
     best = torch.full((M, 1), -3.0e38, dtype=torch.float32, device=cuda)
     bidx = torch.zeros((M, 1), dtype=torch.int32, device=cuda)
-    ops.gemm_nt_group_argmax(dev(a), dev(as_), dev(b), dev(bs), best, bidx, group)
+    tb = torch.zeros((N, 1024 + 16 * padded), dtype=torch.int8, device=cuda)[:, :1024]
+    tb.copy_(dev(b))
+    ops.gemm_nt_group_argmax(dev(a), dev(as_), tb, dev(bs), best, bidx, group)
     ref = oracle.gemm_nt_group(a, as_, b, bs, group)
     assert host(bidx)[:, 0].tolist() == [int(i) for i in np.argmax(ref, axis=1)]
     assert bits_equal(host(best)[:, 0], ref.max(axis=1))
