@@ -135,9 +135,11 @@ q3::GemvArgs to_gemv(const q3::GemmArgs &g);
 // columns, 9 rows 47.2 / 33.9), as long as its keys (one per 128 columns and
 // row) fit the 4 MiB workspace.  But K = 1024 in groups of 128 dequantises twice
 // as often on the tiles: 65536 columns, 9 rows 17.2 / 16.4, 100096 columns 23.7
-// / 24.7, 16 rows 24.9 / 24.7, 151936 columns 31.2 / 33.3 and 32.7 / 33.2.
+// / 24.7, 16 rows 24.9 / 24.7, 151936 columns 31.2 / 33.3 and 32.7 / 33.2; from
+// there on the GEMV up to 16 rows while its keys (one per 64 columns) fit too.
 bool use_gemv(const q3::GemmArgs &g) {
-  const bool tile_from_9 = g.K != 1024 || g.group != 128 || g.N < 98304;
+  const bool tile_from_9 = g.K != 1024 || g.group != 128 || g.N < 98304 ||
+                           static_cast<int64_t>(g.N / 64) * g.M > (1 << 19);
   if (g.epi == q3::EPI_ARGMAX && g.M > (tile_from_9 ? 8 : 16) && g.N >= 65536 &&
       static_cast<int64_t>(g.N / 128) * g.M <= (1 << 19))
     return false;

@@ -112,3 +112,27 @@ def test_argmax_wide_routes(cuda, N, group, M):
     ref = oracle.gemm_nt_group(a, as_, b, bs, group)
     assert host(bidx)[:, 0].tolist() == [int(i) for i in np.argmax(ref, axis=1)]
     assert bits_equal(host(best)[:, 0], ref.max(axis=1))
+
+
+def test_argmax_key_limit(cuda):
+    """16 rows over more columns than the GEMV has keys for (one per 64
+    columns), but the tile kernel (one per 128): as two calls over halves."""
+    M, N, K, group = 16, (1 << 21) + 256, 1024, 128
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(21)
+    b = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=cuda, generator=gen)
+    bs = torch.rand((N, 1), device=cuda, generator=gen)
+    a = torch.randint(-127, 128, (M, K), dtype=torch.int8, device=cuda, generator=gen)
+    as_ = torch.rand((M, K // group), device=cuda, generator=gen)
+
+    def argmax(lo, hi):
+        best = torch.full((M, 1), -3.0e38, dtype=torch.float32, device=cuda)
+        bidx = torch.zeros((M, 1), dtype=torch.int32, device=cuda)
+        ops.gemm_nt_group_argmax(a, as_, b[lo:hi], bs[lo:hi], best, bidx, group)
+        return host(best)[:, 0], host(bidx)[:, 0] + lo
+
+    best, bidx = argmax(0, N)
+    half = N // 2
+    (b0, i0), (b1, i1) = argmax(0, half), argmax(half, N)
+    assert bits_equal(best, np.maximum(b0, b1))
+    assert np.array_equal(bidx, np.where(b1 > b0, i1, i0))
