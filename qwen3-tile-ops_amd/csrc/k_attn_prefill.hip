@@ -39,14 +39,17 @@
 // of a two-chunk LDS ring, the K operand rows and ks | vs straight into
 // registers.
 //
-// What bounds it: VALU issue (about 620 instructions per wave, block and 16
-// rows; the exps are 5 % of the time) and, with few workgroups, the serial
-// phases of a step (4.2 us for 8 blocks on an otherwise idle CU).  K rows and
-// scales of a chunk are loaded under phases 2 to 4 of the chunk before (after
-// phase 3 they cost 27 % of a long walk).  512 rows x 512 keys 15.2 us, 512 x
-// 3500 78 us, 301 x 2349 50 us, 2048 x 2048 112 us (before the early loads,
-// 32-bit offsets, immediate LDS offsets, the approximate reciprocal and the
-// corr = 1 path: 15.4, 94, 60 and 129 us).
+// What bounds it: VALU issue (620-660 instructions per wave, block and 16 rows;
+// a busy CU issues one in 79 % of its cycles at 2048 x 2048, 54 % at 301 x 2349,
+// 52 % at 512 x 512 by counters) and, with few workgroups, the serial phases of a
+// step (4.2 us for 8 blocks on an otherwise idle CU).  No one part carries it:
+// with the exps replaced by one FMA each, 512 x 512 takes 4 % less and the long
+// walks 11-12 %, without the quantisation of P 1-5 %, without the arithmetic of
+// phase 4 5-10 %.  K rows and scales of a chunk are loaded under phases 2 to 4 of
+// the chunk before (after phase 3 they cost 27 % of a long walk).  512 rows x 512
+// keys 15.2 us, 512 x 3500 78 us, 301 x 2349 50 us, 2048 x 2048 112 us (before
+// the early loads, 32-bit offsets, immediate LDS offsets, the approximate
+// reciprocal and the corr = 1 path: 15.4, 94, 60 and 129 us).
 //
 // Layouts (lane = lc + 16 lg):
 //   S^T_j = K_j . Q^T with v_mfma_i32_16x16x64_i8, keys as the M dimension:
@@ -326,8 +329,8 @@ __global__ void __launch_bounds__(Cfg<NI>::NW * 64, 4) attn_prefill_kernel(AttnA
   load_sc(0, page);
   page = page_of(1);
   if (threadIdx.x == 0) stage_exp2_table(L.etab);
-  // Q row lc of item A / B as the B operand, [item][64-byte k-step]; loaded
-  // with each chunk's K rows so that it is not live through phases 3-4
+  // Q row lc of item A / B as the B operand, [item][64-byte k-step], for the
+  // whole walk
   v4i qop[2][2];
   float qsv[2];
   auto load_q = [&](int g) {

@@ -96,7 +96,7 @@ struct q3_model {
   double kt_ms[Q3_KT_COUNT] = {};              // folded totals
   uint32_t kt_n[Q3_KT_COUNT] = {};             // calls timed (a call may be several launches)
   // decode: workgroups that prefetch the next kernels' weights during the
-  // attention kernel (Q3_DECODE_PREFETCH_WGS, default 176; 0 disables)
+  // attention kernel (Q3_DECODE_PREFETCH_WGS, default 120; 0 disables)
   int pf_wgs;
   // decode: O projection folded into the attention kernel
   // (Q3_DECODE_FUSE_OPROJ, default 1; 0 runs it as its own GEMV)
