@@ -181,14 +181,6 @@ __device__ __forceinline__ Item make_item(const PreArgs &a, int qb, int kv_len) 
   return it;
 }
 
-// quant_rcp (q3_device.h) for x >= 0 (P * vs): the NaN of 0 * inf goes to
-// +0 through the max.
-__device__ __forceinline__ int quant_rcp_pos(float x, double y) {
-  float q = __double2float_rn(__dmul_rn(static_cast<double>(x), y));
-  q = fmaxf(q, 0.0f);
-  return static_cast<int>(fminf(rintf(q), 127.0f));
-}
-
 __device__ __forceinline__ uint32_t pack4(int b0, int b1, int b2, int b3) {
   return (static_cast<uint32_t>(b0) & 0xffu) | ((static_cast<uint32_t>(b1) & 0xffu) << 8) |
          ((static_cast<uint32_t>(b2) & 0xffu) << 16) | (static_cast<uint32_t>(b3) << 24);

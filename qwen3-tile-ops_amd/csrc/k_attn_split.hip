@@ -423,13 +423,27 @@ __global__ void __launch_bounds__(kWaves * 64) split_chunk_kernel(SplitArgs a) {
       }
       const float pm = __fmul_rn(fold_max(pmx), inv127());
       const double y = rcp64(pm);
-      uint32_t w8[2];
+      // (as k_attn_prefill.hip quantises: without clamps while every row's pm is
+      // normal, so that a negative vs, which no quantisation gives, comes out
+      // the same on both routes)
+      uint32_t q8[2][4], w8[2];
+      if (__builtin_amdgcn_ballot_w64(!(pm >= 1.17549435e-38f)) == 0) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        w8[kt] = 0;
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w8[kt] |= (static_cast<uint32_t>(quant_rcp(p[kt][i], y)) & 0xffu) << (8 * i);
+          for (int i = 0; i < 4; ++i)
+            q8[kt][i] = static_cast<uint32_t>(
+                static_cast<int>(rintf(__double2float_rn(__dmul_rn(static_cast<double>(p[kt][i]), y)))));
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) q8[kt][i] = static_cast<uint32_t>(quant_rcp_pos(p[kt][i], y));
       }
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        w8[kt] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q8[kt][3], q8[kt][2], 0x0c0c0400u),
+                                       __builtin_amdgcn_perm(q8[kt][1], q8[kt][0], 0x0c0c0400u), 0x05040100u);
       if (lg == 0 && lc < nr) {
         a.ws_psum[wb] = __fadd_rn(ts[0], ts[1]);
         a.ws_nmm[wb] = nmm;

@@ -289,6 +289,13 @@ __device__ __forceinline__ int quant_rcp(float x, double y) {
   return static_cast<int>(r);
 }
 
+// quant_rcp for x >= 0 (P * vs): the NaN of 0 * inf goes to +0 through the max.
+__device__ __forceinline__ int quant_rcp_pos(float x, double y) {
+  float q = __double2float_rn(__dmul_rn(static_cast<double>(x), y));
+  q = fmaxf(q, 0.0f);
+  return static_cast<int>(fminf(rintf(q), 127.0f));
+}
+
 // ---- lane exchanges in VALU (no LDS round trip) -----------------------
 // lane_xor<M>(x): lane i receives x of lane i ^ M.  M = 1, 2: DPP quad_perm;
 // M = 4: quad_perm [3,2,1,0] then row_half_mirror (i -> (i ^ 3) ^ 7);

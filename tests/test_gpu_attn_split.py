@@ -187,11 +187,12 @@ def test_split_chunk_matches_tile_walk(cuda, monkeypatch):
                 assert bits_equal(a, b), (what, describe_diff(a, b))
 
 
-@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
-def test_split_special_scales(cuda, monkeypatch, value):
-    """Rows whose scores are infinite or NaN (K scales of the pool) come out
-    as from the kernels that take the same rows without the split: a chunk's
-    with scale 0, a decoding row's with scale NaN."""
+@pytest.mark.parametrize("which", ["k", "v"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, -0.02, 1e-44])
+def test_split_special_scales(cuda, monkeypatch, which, value):
+    """Rows over infinite, NaN, negative or subnormal scales in the pool come
+    out as from the kernels that take the same rows without the split; with
+    infinite or NaN scores a chunk's row has scale 0, a decoding row's NaN."""
     lay = Layout(ModelShape(layers=1, vocab=1024, seq=64, max_seq=1024))
     blob = init_random_blob(lay, InitConfig(n_prompt=1, n_gen=0, mode=0))
     rng = np.random.default_rng(17)
@@ -201,7 +202,7 @@ def test_split_special_scales(cuda, monkeypatch, value):
         n = ms * lay.kv_width
         blob[at:at + n] = rng.integers(-127, 128, n, dtype=np.int8).view(np.uint8)
         sc = rng.uniform(0.002, 0.03, ms * lay.kv_heads).astype(np.float32)
-        if off == 0:
+        if (off == 0) == (which == "k"):
             sc.reshape(-1, lay.kv_heads)[40::300, ::2] = value
         blob[at + o["kKV_SOFF"]:at + o["kKV_SOFF"] + 4 * sc.size] = sc.view(np.uint8)
     ids = rng.integers(0, 1024, ms).astype(np.int32)
@@ -226,7 +227,8 @@ def test_split_special_scales(cuda, monkeypatch, value):
         if split == "1":
             w8, ws = got[("0", *what)]
             assert np.array_equal(o8, w8) and np.array_equal(os_, ws, equal_nan=True), what
-    assert np.isnan(got["1", 1000, 1][1]).any() and not np.isnan(got["1", 960, 64][1]).any()
+    if which == "k" and not np.isfinite(value):
+        assert np.isnan(got["1", 1000, 1][1]).any() and not np.isnan(got["1", 960, 64][1]).any()
 
 
 @pytest.mark.parametrize("split", ["0", "1"])
